@@ -1151,7 +1151,10 @@ using namespace eg;
 extern "C" size_t eg_attn_gqa_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads,
                                               int64_t seq, int64_t head_dim) {
   if (batch <= 0 || heads <= 0 || seq <= 0 || kv_heads <= 0) return 0;
-  return attn_delta_bytes(batch * heads, seq) + attn_part_bytes(batch * kv_heads, seq, head_dim);
+  // the dtype is not known here: the larger of the MFMA and the generic kernels' slabs
+  return attn_delta_bytes(batch * heads, seq) +
+         std::max(attn_part_bytes(batch * kv_heads, seq, head_dim),
+                  attn_generic_part_bytes(batch, heads, kv_heads, seq, head_dim));
 }
 
 extern "C" size_t eg_attn_workspace_bytes(int64_t batch, int64_t heads, int64_t seq,
@@ -1195,8 +1198,9 @@ extern "C" int eg_attn_gqa_bwd(const void* dout, const void* q, const void* k, c
   hipStream_t st = as_stream(stream);
   float* delta = (float*)workspace;
   if (!mfma_shape(head_dim, dtype))
-    return attn_generic_bwd(dout, q, k, v, o, lse, dq, dk, dv, delta, batch, heads, kv_heads, seq,
-                            head_dim, scale, dtype, st);
+    return attn_generic_bwd(dout, q, k, v, o, lse, dq, dk, dv, delta,
+                            (float*)((char*)delta + attn_delta_bytes(batch * heads, seq)), batch,
+                            heads, kv_heads, seq, head_dim, scale, dtype, st);
   if (!attn_aligned({dout, q, k, v, o, dq, dk, dv})) {
     set_error("eg_attn_bwd: tensors must be 16-byte aligned");
     return 1;

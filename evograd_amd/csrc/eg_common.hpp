@@ -267,20 +267,18 @@ int gemm_logits_softmax_launch(const void* x, const void* w, void* e, int64_t m,
                                const int64_t* target, float* hstats, float* tlogit, int dtype,
                                hipStream_t st, const char* name);
 
-// Causal GQA attention on plain fp32 arithmetic (attn_generic.hip) for the shapes
-// the MFMA kernels do not take: any dtype, even head_dim <= 128. Arguments as
+// Causal GQA attention in fp32 arithmetic (attn_generic.hip) for the shapes the 16-bit
+// MFMA kernels do not take: any dtype, even head_dim <= 128. Arguments as
 // eg_attn_gqa_fwd / eg_attn_gqa_bwd, already validated; delta is the backward's
-// fp32 [B, H, S] workspace. With tables rc, rs (fp32 [S, D]) the forward rotates q
-// as it loads it (k already rotated) and the backward takes the rotated q, k and
-// writes dq, dk for the pre-rotation ones.
+// fp32 [B, H, S] workspace and part its attn_generic_part_bytes of slabs.
+size_t attn_generic_part_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t S, int64_t D);
 int attn_generic_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B,
                      int64_t H, int64_t Hkv, int64_t S, int64_t D, float scale, int dtype,
-                     hipStream_t st, const float* rc = nullptr, const float* rs = nullptr);
+                     hipStream_t st);
 int attn_generic_bwd(const void* dout, const void* q, const void* k, const void* v,
                      const void* o, const float* lse, void* dq, void* dk, void* dv, float* delta,
-                     int64_t B, int64_t H, int64_t Hkv, int64_t S, int64_t D, float scale,
-                     int dtype, hipStream_t st, const float* rc = nullptr,
-                     const float* rs = nullptr);
+                     float* part, int64_t B, int64_t H, int64_t Hkv, int64_t S, int64_t D,
+                     float scale, int dtype, hipStream_t st);
 
 // The RoPE launch behind eg_rope (rope.hip), for entry points that rotate as one
 // step of a longer launch sequence: arguments as eg_rope's, already validated.

@@ -228,7 +228,8 @@ int eg_attn_gqa_fwd(const void* q, const void* k, const void* v, void* o, float*
  * heads, seq] (heads = query heads), rounded up to 256 bytes; then, for shapes with
  * fewer than 1024 (kv head, 128-key block) pairs, where the dK/dV walk over the
  * query tiles is split into parts (at most 8, a choice of the shape alone), the
- * parts' fp32 sums: 2 x parts x batch x kv_heads x seq x head_dim x 4 bytes.
+ * parts' fp32 sums: 2 x parts x batch x kv_heads x seq x head_dim x 4 bytes (head
+ * sizes other than 64 and 128: the same with fewer than 512 pairs of 16-key blocks).
  * eg_attn_workspace_bytes (for eg_attn_bwd) is this with kv_heads = heads. */
 size_t eg_attn_gqa_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads,
                                    int64_t seq, int64_t head_dim);
