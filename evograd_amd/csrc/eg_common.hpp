@@ -253,6 +253,14 @@ int gemm_launch(const void* a, const void* b, void* c, int64_t m, int64_t n, int
                 const void* r = nullptr, int64_t ldr = 0, bool r_f32 = false,
                 void* ws = nullptr, size_t ws_bytes = 0);
 
+// The fp32 product behind gemm_launch (gemm_f32.hip): arguments as gemm_launch's, already
+// validated; a workspace of gemm_f32_workspace_bytes lets a small output split k.
+size_t gemm_f32_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int gemm_f32_launch(const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k,
+                    int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
+                    int64_t b_rows, hipStream_t st, const char* name, const float* r, int64_t ldr,
+                    void* ws, size_t ws_bytes);
+
 // The logits product of the fused linear cross entropy with its softmax terms
 // formed in the epilogue (gemm_kernel.hpp), 16-bit operands only: for logits = x w^T
 // (x [m][ldx] and w [n][ldw] both k-contiguous, k % 64 == 0) it writes, per

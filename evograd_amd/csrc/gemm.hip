@@ -115,23 +115,9 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
       set_error("%s: a leading dimension is smaller than its row", name);
       return 1;
     }
-    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-    if (grid.y > 65535) {
-      set_error("%s: M too large for the fp32 path", name);
-      return 1;
-    }
-    auto go32 = [&](auto akc, auto bkc) {
-      EG_LAUNCH((gemm_f32_kernel<decltype(akc)::value, decltype(bkc)::value>), grid, dim3(256),
-                0, st, (const float*)A, (const float*)B, (float*)C, (int)M, (int)N, (int)K, lda,
-                ldb, ldc, a_rows, b_rows, (const float*)R, ldr);
-      return check_launch(name);
-    };
-    using TT = std::true_type;
-    using FF = std::false_type;
-    if (a_kc && b_kc) return go32(TT{}, TT{});
-    if (a_kc) return go32(TT{}, FF{});
-    if (b_kc) return go32(FF{}, TT{});
-    return go32(FF{}, FF{});
+    return gemm_f32_launch((const float*)A, (const float*)B, (float*)C, M, N, K, lda, ldb, ldc,
+                           a_kc, b_kc, a_rows, b_rows, st, name, (const float*)R, ldr, ws,
+                           ws_bytes);
   }
   if (dtype != EG_BF16 && dtype != EG_F16) {
     set_error("%s: operands must be fp32, bf16 or fp16", name);
@@ -303,6 +289,7 @@ int gemm_logits_softmax_launch(const void* x, const void* w, void* e, int64_t M,
 using namespace eg;
 
 extern "C" size_t eg_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int dtype) {
+  if (dtype == EG_F32) return gemm_f32_workspace_bytes(m, n, k);
   if (dtype != EG_BF16 && dtype != EG_F16) return 0;
   return gemm_workspace_bytes(m, n, k);
 }

@@ -794,56 +794,6 @@ void gemm_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
   }
 }
 
-// fp32 operands (no fp32 MFMA path is worth its registers here): a plain tiled
-// product, 64 x 64 outputs per 256-thread workgroup, 4 x 4 per thread, 16-deep
-// k slices staged in LDS with every element bounds-checked. Used for fp32 inputs
-// of the fused linear cross entropy.
-template <bool AKC, bool BKC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A,
-                                                       const float* __restrict__ B,
-                                                       float* C, int M, int N, int K,
-                                                       int64_t lda, int64_t ldb, int64_t ldc,
-                                                       int64_t a_rows, int64_t b_rows,
-                                                       const float* R, int64_t ldr) {
-  __shared__ float As[16][65], Bs[16][65];
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int kk = e / 64, mm = e % 64;
-      const int64_t k = k0 + kk, m = m0 + mm, n = n0 + mm;
-      float av = 0.f, bv = 0.f;
-      if (k < K && m < M) {
-        const int64_t r = AKC ? m : k;
-        if (r < a_rows) av = AKC ? A[m * lda + k] : A[k * lda + m];
-      }
-      if (k < K && n < N) {
-        const int64_t r = BKC ? n : k;
-        if (r < b_rows) bv = BKC ? B[n * ldb + k] : B[k * ldb + n];
-      }
-      As[kk][mm] = av;
-      Bs[kk][mm] = bv;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += As[kk][ty * 4 + i] * Bs[kk][tx * 4 + j];
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = m0 + ty * 4 + i, n = n0 + tx * 4 + j;
-      if (m < M && n < N)
-        C[(int64_t)m * ldc + n] = R ? acc[i][j] + R[(int64_t)m * ldr + n] : acc[i][j];
-    }
-}
-
 // Split-K reduction: c[m][n] = r[m][n] + sum over s (in order) of part[s][m][n],
 // rounded once to TC. Four consecutive columns per thread when N % 4 == 0.
 template <typename TC, int V>

@@ -771,8 +771,12 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
         }
         if (int rc = check_launch(name)) return rc;
       }
+      // fp32 inputs: the chunk's logits are spent, their buffer holds split-k partials
+      void* gws = dtype == EG_F32 ? (void*)logits : nullptr;
+      const size_t gws_bytes = dtype == EG_F32 ? L.logits : 0;
       if (int rc = gemm_launch(dlp, weight, (T*)dx + r0 * hidden, n, hidden, L.vp, L.vp, hidden,
-                               hidden, true, false, n, vocab, dtype, dtype, st, name))
+                               hidden, true, false, n, vocab, dtype, dtype, st, name, nullptr, 0,
+                               false, gws, gws_bytes))
         return rc;
       // dW = sum over chunks of dl_c^T x_c: into dW directly (one chunk, or fp32
       // inputs), else into the fp32 sum, the last chunk rounding it once into dW
@@ -781,7 +785,7 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
       const void* res = first ? nullptr : (acc ? (const void*)acc : dweight);
       if (int rc = gemm_launch(dlp, xc, out, vocab, hidden, n, L.vp, hidden, hidden, false,
                                false, n, n, dtype, out == acc ? EG_F32 : dtype, st, name, res,
-                               hidden, acc != nullptr))
+                               hidden, acc != nullptr, gws, gws_bytes))
         return rc;
     }
     EG_LAUNCH((xent_mean_kernel<float>), dim3(1), dim3(kMeanBlock), 0, st, target, rowloss, loss,

@@ -374,8 +374,9 @@ int eg_scale_copy(const void* src, int src_dtype, void* dst, int dst_dtype, int6
  * split k over workgroups when `workspace` holds at least
  * eg_gemm_workspace_bytes(m, n, k, dtype) bytes (else, or with workspace NULL, they
  * run unsplit): each k range writes an fp32 partial, and a second pass sums them in
- * a fixed order, adds r and rounds c once. So do the tiles of a last wave that is at most half full (more than 256
- * tiles). The split depends on the shape only, so results are bitwise repeatable. */
+ * a fixed order, adds r and rounds c once. So do the tiles of a last wave that is at
+ * most half full (more than 256 tiles), and fp32 products of fewer than 256 tiles of
+ * 32 x 32 (at most 8 ranges). The split depends on the shape only, so results are bitwise repeatable. */
 size_t eg_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int dtype);
 int eg_gemm(const void* a, const void* b, void* c, const void* r, int64_t m, int64_t n,
             int64_t k, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldr, int a_k_contiguous,
