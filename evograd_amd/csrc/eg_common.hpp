@@ -139,6 +139,54 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&in)[V
   else store_f32<T, VEC>(p, in);
 }
 
+// Ragged rows: 16-byte packs of rows that start at any element (a row width that is no
+// multiple of the pack, or an unaligned base). gfx950's global accesses take any element
+// alignment, at the cost of touching one more cache line per wave. The last pack of a row
+// starts VEC elements before the row's end, so it stays inside the row and overlaps the
+// pack before it; its elements below `lo` belong to that one and are neither counted nor
+// stored. Rows narrower than one pack take the element paths.
+struct RaggedPack {
+  int c, lo;  // first column; first element of the pack's own
+};
+template <int VEC>
+__device__ __forceinline__ RaggedPack ragged_pack(int c, int cols) {
+  const int c0 = min(c, cols - VEC);
+  return {c0, c - c0};
+}
+// NT: with the non-temporal hint (16-byte packs only, as in load_vec).
+template <typename T, int VEC, bool NT>
+__device__ __forceinline__ void load_ragged(const T* __restrict__ p, float (&out)[VEC]) {
+  typedef unsigned int words __attribute__((ext_vector_type(sizeof(T) * VEC / 4)));
+  typedef words __attribute__((aligned(sizeof(T)))) any_words;
+  const any_words* a = reinterpret_cast<const any_words*>(p);
+  words raw;
+  if constexpr (NT && sizeof(T) * VEC == 16) raw = __builtin_nontemporal_load(a);
+  else raw = *a;
+  Pack<T, VEC> pk;
+  __builtin_memcpy(&pk, &raw, sizeof(raw));
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) out[i] = to_f32(pk.v[i]);
+}
+template <typename T, int VEC, bool NT>
+__device__ __forceinline__ void store_ragged(T* __restrict__ p, int lo, const float (&in)[VEC]) {
+  typedef unsigned int words __attribute__((ext_vector_type(sizeof(T) * VEC / 4)));
+  typedef words __attribute__((aligned(sizeof(T)))) any_words;
+  Pack<T, VEC> pk;
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) pk.v[i] = from_f32<T>(in[i]);
+  if (lo == 0) {
+    words raw;
+    __builtin_memcpy(&raw, &pk, sizeof(raw));
+    any_words* a = reinterpret_cast<any_words*>(p);
+    if constexpr (NT && sizeof(T) * VEC == 16) __builtin_nontemporal_store(raw, a);
+    else *a = raw;
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      if (i >= lo) p[i] = pk.v[i];
+  }
+}
+
 // ------------------------------------------------------------- reductions
 struct SumOp {
   __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }

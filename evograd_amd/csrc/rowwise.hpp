@@ -17,10 +17,36 @@ constexpr int kUnroll = 4;  // packs in flight per thread
 // max is replaced by 0 so that exp(x - ref) stays defined.
 __device__ __forceinline__ float lse_ref(float m) { return __builtin_isinf(m) ? 0.f : m; }
 
+// The pack at column c (below cols) of a row; of a ragged row's last pack, the elements
+// that are not its own become `fill`.
+template <typename T, int VEC, bool NT, bool RAG>
+__device__ __forceinline__ void load_pack(const T* __restrict__ row, int c, int cols, float fill,
+                                          float (&v)[VEC]) {
+  if constexpr (RAG) {
+    const RaggedPack p = ragged_pack<VEC>(c, cols);
+    load_ragged<T, VEC, NT>(row + p.c, v);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) v[i] = i < p.lo ? fill : v[i];
+  } else {
+    load_vec<T, VEC, NT>(row + c, v);
+  }
+}
+// The same pack's store.
+template <typename T, int VEC, bool NT, bool RAG>
+__device__ __forceinline__ void store_pack(T* __restrict__ row, int c, int cols,
+                                           const float (&v)[VEC]) {
+  if constexpr (RAG) {
+    const RaggedPack p = ragged_pack<VEC>(c, cols);
+    store_ragged<T, VEC, NT>(row + p.c, p.lo, v);
+  } else {
+    store_vec<T, VEC, NT>(row + c, v);
+  }
+}
+
 // logsumexp of the row xr[0 .. cols) in fp32, returned to every thread: an online
 // (max, sum of exp2) per thread, then one max and one sum over the workgroup.
-// `red` holds BLOCK / 64 floats of LDS.
-template <typename T, int VEC, int BLOCK, bool NT>
+// `red` holds BLOCK / 64 floats of LDS. RAG: the row is ragged (eg_common.hpp).
+template <typename T, int VEC, int BLOCK, bool NT, bool RAG = false>
 __device__ __forceinline__ float row_lse(const T* __restrict__ xr, int cols, float* red) {
   constexpr int STEP = BLOCK * VEC;
   float m = -INFINITY;  // running max of this thread's elements
@@ -31,7 +57,7 @@ __device__ __forceinline__ float row_lse(const T* __restrict__ xr, int cols, flo
     for (int u = 0; u < kUnroll; ++u) {
       const int c = base + u * STEP;
       if (c < cols) {
-        load_vec<T, VEC, NT>(xr + c, v[u]);
+        load_pack<T, VEC, NT, RAG>(xr, c, cols, -INFINITY, v[u]);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[u][i] = -INFINITY;
@@ -66,7 +92,7 @@ __device__ __forceinline__ float row_lse(const T* __restrict__ xr, int cols, flo
 }
 
 // sum(a * b) over the row, in fp32, returned to every thread.
-template <typename T, int VEC, int BLOCK, bool NT>
+template <typename T, int VEC, int BLOCK, bool NT, bool RAG = false>
 __device__ __forceinline__ float row_dot(const T* __restrict__ a, const T* __restrict__ b,
                                          int cols, float* red) {
   constexpr int STEP = BLOCK * VEC;
@@ -77,8 +103,8 @@ __device__ __forceinline__ float row_dot(const T* __restrict__ a, const T* __res
     for (int u = 0; u < kUnroll; ++u) {
       const int c = base + u * STEP;
       if (c < cols) {
-        load_vec<T, VEC, NT>(a + c, va[u]);
-        load_vec<T, VEC, NT>(b + c, vb[u]);
+        load_pack<T, VEC, NT, RAG>(a, c, cols, 0.f, va[u]);
+        load_pack<T, VEC, NT, RAG>(b, c, cols, 0.f, vb[u]);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) va[u][i] = vb[u][i] = 0.f;

@@ -12,7 +12,8 @@
 // (softmax_fwd_lds / softmax_bwd_lds), so both passes read HBM once. Wider rows take a
 // two-read path: the row's logsumexp
 // (forward) or sum(dy * y) (backward) in one read, then y = exp(x - lse) or
-// dx = y * (dy - sum) in a second read and the write.
+// dx = y * (dy - sum) in a second read and the write. Rows that are no multiple of a
+// 16-byte pack are read in unaligned packs (RAG; eg_common.hpp).
 #include "rowwise.hpp"
 
 namespace eg {
@@ -26,10 +27,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, int
 }
 constexpr int kNtAux = 2;  // buffer access cache policy: non-temporal
 
-template <typename T, int VEC, int ITEMS, int BLOCK, bool NT>
+template <typename T, int VEC, int ITEMS, int BLOCK, bool NT, bool RAG>
 __device__ __forceinline__ void load_row(const T* __restrict__ row, int cols, float fill,
                                          float (&v)[ITEMS][VEC]) {
-  if constexpr (NT) {  // 16-byte packs
+  if constexpr (NT && !RAG) {  // 16-byte packs
     const __amdgpu_buffer_rsrc_t rs = row_rsrc(row, cols * (int)sizeof(T));
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -47,7 +48,7 @@ __device__ __forceinline__ void load_row(const T* __restrict__ row, int cols, fl
     for (int it = 0; it < ITEMS; ++it) {
       const int c = (it * BLOCK + (int)threadIdx.x) * VEC;
       if (c < cols) {
-        load_vec<T, VEC, NT>(row + c, v[it]);
+        rowwise::load_pack<T, VEC, NT, RAG>(row, c, cols, fill, v[it]);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[it][i] = fill;
@@ -56,10 +57,10 @@ __device__ __forceinline__ void load_row(const T* __restrict__ row, int cols, fl
   }
 }
 
-template <typename T, int VEC, int ITEMS, int BLOCK, bool NT>
+template <typename T, int VEC, int ITEMS, int BLOCK, bool NT, bool RAG>
 __device__ __forceinline__ void store_row(T* __restrict__ row, int cols,
                                           const float (&v)[ITEMS][VEC]) {
-  if constexpr (NT) {
+  if constexpr (NT && !RAG) {
     const __amdgpu_buffer_rsrc_t rs = row_rsrc(row, cols * (int)sizeof(T));
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -76,18 +77,18 @@ __device__ __forceinline__ void store_row(T* __restrict__ row, int cols,
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int c = (it * BLOCK + (int)threadIdx.x) * VEC;
-      if (c < cols) store_vec<T, VEC, NT>(row + c, v[it]);
+      if (c < cols) rowwise::store_pack<T, VEC, NT, RAG>(row, c, cols, v[it]);
     }
   }
 }
 
-template <typename T, int VEC, int ITEMS, int BLOCK, bool NT>
+template <typename T, int VEC, int ITEMS, int BLOCK, bool NT, bool RAG>
 __global__ __launch_bounds__(BLOCK) void softmax_fwd_reg(const T* __restrict__ x,
                                                          T* __restrict__ y, int cols) {
   __shared__ float lds[BLOCK / kWave];
   const int64_t off = (int64_t)blockIdx.x * cols;
   float v[ITEMS][VEC];
-  load_row<T, VEC, ITEMS, BLOCK, NT>(x + off, cols, -INFINITY, v);
+  load_row<T, VEC, ITEMS, BLOCK, NT, RAG>(x + off, cols, -INFINITY, v);
   float m = -INFINITY;
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
@@ -112,18 +113,18 @@ __global__ __launch_bounds__(BLOCK) void softmax_fwd_reg(const T* __restrict__ x
   for (int it = 0; it < ITEMS; ++it)
 #pragma unroll
     for (int i = 0; i < VEC; ++i) v[it][i] *= inv;
-  store_row<T, VEC, ITEMS, BLOCK, NT>(y + off, cols, v);
+  store_row<T, VEC, ITEMS, BLOCK, NT, RAG>(y + off, cols, v);
 }
 
-template <typename T, int VEC, int ITEMS, int BLOCK, bool NT>
+template <typename T, int VEC, int ITEMS, int BLOCK, bool NT, bool RAG>
 __global__ __launch_bounds__(BLOCK) void softmax_bwd_reg(const T* __restrict__ y,
                                                          const T* __restrict__ dy,
                                                          T* __restrict__ dx, int cols) {
   __shared__ float lds[BLOCK / kWave];
   const int64_t off = (int64_t)blockIdx.x * cols;
   float yv[ITEMS][VEC], gv[ITEMS][VEC];
-  load_row<T, VEC, ITEMS, BLOCK, NT>(y + off, cols, 0.f, yv);
-  load_row<T, VEC, ITEMS, BLOCK, NT>(dy + off, cols, 0.f, gv);
+  load_row<T, VEC, ITEMS, BLOCK, NT, RAG>(y + off, cols, 0.f, yv);
+  load_row<T, VEC, ITEMS, BLOCK, NT, RAG>(dy + off, cols, 0.f, gv);
   float d = 0.f;
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
@@ -134,12 +135,12 @@ __global__ __launch_bounds__(BLOCK) void softmax_bwd_reg(const T* __restrict__ y
   for (int it = 0; it < ITEMS; ++it)
 #pragma unroll
     for (int i = 0; i < VEC; ++i) gv[it][i] = yv[it][i] * (gv[it][i] - d);
-  store_row<T, VEC, ITEMS, BLOCK, NT>(dx + off, cols, gv);
+  store_row<T, VEC, ITEMS, BLOCK, NT, RAG>(dx + off, cols, gv);
 }
 
 // ---- wide rows: one read for the row statistic (lse, or sum(dy * y)), a second
 // read to write, each with kUnroll 16-byte packs in flight per thread.
-template <typename T, int VEC, int BLOCK, bool NT>
+template <typename T, int VEC, int BLOCK, bool NT, bool RAG>
 __global__ __launch_bounds__(BLOCK) void softmax_fwd_loop(const T* __restrict__ x,
                                                           T* __restrict__ y, int cols) {
   __shared__ float lds[BLOCK / kWave];
@@ -151,13 +152,13 @@ __global__ __launch_bounds__(BLOCK) void softmax_fwd_loop(const T* __restrict__ 
   // The statistic's read is a temporal load, so that the rows in flight (256 KB
   // each at bf16 x 128K columns) can serve the second read from the device cache;
   // the second read is the last use.
-  const float ll = rowwise::row_lse<T, VEC, BLOCK, false>(xr, cols, lds) * rowwise::kLog2e;
+  const float ll = rowwise::row_lse<T, VEC, BLOCK, false, RAG>(xr, cols, lds) * rowwise::kLog2e;
   for (int base = (int)threadIdx.x * VEC; base < cols; base += STEP * rowwise::kUnroll) {
     float v[rowwise::kUnroll][VEC];
 #pragma unroll
     for (int u = 0; u < rowwise::kUnroll; ++u) {
       const int c = base + u * STEP;
-      if (c < cols) load_vec<T, VEC, NT>(xr + c, v[u]);
+      if (c < cols) rowwise::load_pack<T, VEC, NT, RAG>(xr, c, cols, 0.f, v[u]);
     }
 #pragma unroll
     for (int u = 0; u < rowwise::kUnroll; ++u) {
@@ -166,13 +167,13 @@ __global__ __launch_bounds__(BLOCK) void softmax_fwd_loop(const T* __restrict__ 
 #pragma unroll
         for (int i = 0; i < VEC; ++i)
           v[u][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[u][i], rowwise::kLog2e, -ll));
-        store_vec<T, VEC, NT>(yr + c, v[u]);
+        rowwise::store_pack<T, VEC, NT, RAG>(yr, c, cols, v[u]);
       }
     }
   }
 }
 
-template <typename T, int VEC, int BLOCK, bool NT>
+template <typename T, int VEC, int BLOCK, bool NT, bool RAG>
 __global__ __launch_bounds__(BLOCK) void softmax_bwd_loop(const T* __restrict__ y,
                                                           const T* __restrict__ dy,
                                                           T* __restrict__ dx, int cols) {
@@ -183,15 +184,15 @@ __global__ __launch_bounds__(BLOCK) void softmax_bwd_loop(const T* __restrict__ 
   const T* __restrict__ gr = dy + off;
   T* __restrict__ dr = dx + off;
   // temporal first read, as in the forward
-  const float d = rowwise::row_dot<T, VEC, BLOCK, false>(yr, gr, cols, lds);
+  const float d = rowwise::row_dot<T, VEC, BLOCK, false, RAG>(yr, gr, cols, lds);
   for (int base = (int)threadIdx.x * VEC; base < cols; base += STEP * rowwise::kUnroll) {
     float a[rowwise::kUnroll][VEC], b[rowwise::kUnroll][VEC];
 #pragma unroll
     for (int u = 0; u < rowwise::kUnroll; ++u) {
       const int c = base + u * STEP;
       if (c < cols) {
-        load_vec<T, VEC, NT>(yr + c, a[u]);
-        load_vec<T, VEC, NT>(gr + c, b[u]);
+        rowwise::load_pack<T, VEC, NT, RAG>(yr, c, cols, 0.f, a[u]);
+        rowwise::load_pack<T, VEC, NT, RAG>(gr, c, cols, 0.f, b[u]);
       }
     }
 #pragma unroll
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(BLOCK) void softmax_bwd_loop(const T* __restrict__ 
       if (c < cols) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) b[u][i] = a[u][i] * (b[u][i] - d);
-        store_vec<T, VEC, NT>(dr + c, b[u]);
+        rowwise::store_pack<T, VEC, NT, RAG>(dr, c, cols, b[u]);
       }
     }
   }
@@ -425,29 +426,29 @@ bool pick_row_config(int64_t npack, Launch&& launch) {
   return false;
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 struct FwdLaunch {
   const T* x; T* y; int64_t rows; int cols; hipStream_t st;
   template <int BLOCK, int ITEMS> bool go() {
-    EG_LAUNCH((softmax_fwd_reg<T, VEC, ITEMS, BLOCK, VEC * sizeof(T) == 16>), dim3((unsigned)rows),
+    EG_LAUNCH((softmax_fwd_reg<T, VEC, ITEMS, BLOCK, VEC * sizeof(T) == 16, RAG>), dim3((unsigned)rows),
                        dim3(BLOCK), 0, st, x, y, cols);
     return true;
   }
 };
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 struct BwdLaunch {
   const T* y; const T* dy; T* dx; int64_t rows; int cols; hipStream_t st;
   template <int BLOCK, int ITEMS> bool go() {
-    EG_LAUNCH((softmax_bwd_reg<T, VEC, ITEMS, BLOCK, VEC * sizeof(T) == 16>), dim3((unsigned)rows),
+    EG_LAUNCH((softmax_bwd_reg<T, VEC, ITEMS, BLOCK, VEC * sizeof(T) == 16, RAG>), dim3((unsigned)rows),
                        dim3(BLOCK), 0, st, y, dy, dx, cols);
     return true;
   }
 };
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG = false>
 void softmax_fwd_vec(const T* x, T* y, int64_t rows, int cols, hipStream_t st) {
-  FwdLaunch<T, VEC> l{x, y, rows, cols, st};
+  FwdLaunch<T, VEC, RAG> l{x, y, rows, cols, st};
   const int64_t npack = (cols + VEC - 1) / VEC;
   // rows of 513-1024 packs: 512 threads of 2 packs (fp32 [*, 4096]: 25.7 against
   // 26.2 us for 256 threads of 4)
@@ -456,20 +457,20 @@ void softmax_fwd_vec(const T* x, T* y, int64_t rows, int cols, hipStream_t st) {
     return;
   }
   if (pick_row_config(npack, l)) return;
-  if constexpr (sizeof(T) == 2 && VEC == 8) {
+  if constexpr (sizeof(T) == 2 && VEC == 8 && !RAG) {
     if (npack <= (int64_t)kFwdRowItems * kFwdRowBlock) {
       EG_LAUNCH((softmax_fwd_lds<T, kFwdRowItems, kFwdRowLds, kFwdRowBlock>), dim3((unsigned)rows),
                 dim3(kFwdRowBlock), 0, st, x, y, cols);
       return;
     }
   }
-  EG_LAUNCH((softmax_fwd_loop<T, VEC, 1024, VEC * sizeof(T) == 16>), dim3((unsigned)rows),
+  EG_LAUNCH((softmax_fwd_loop<T, VEC, 1024, VEC * sizeof(T) == 16, RAG>), dim3((unsigned)rows),
             dim3(1024), 0, st, x, y, cols);
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG = false>
 void softmax_bwd_vec(const T* y, const T* dy, T* dx, int64_t rows, int cols, hipStream_t st) {
-  BwdLaunch<T, VEC> l{y, dy, dx, rows, cols, st};
+  BwdLaunch<T, VEC, RAG> l{y, dy, dx, rows, cols, st};
   const int64_t npack = (cols + VEC - 1) / VEC;
   // rows of 513-1024 packs: 512 threads of 2 packs, as in the forward (fp32
   // [4096, 4096], interleaved: 33.4 against 34.1 us for 256 threads of 4)
@@ -477,16 +478,28 @@ void softmax_bwd_vec(const T* y, const T* dy, T* dx, int64_t rows, int cols, hip
     l.template go<512, 2>();
     return;
   }
-  if (pick_row_config(npack, l)) return;
-  if constexpr (sizeof(T) == 2 && VEC == 8) {
+  // ragged 16-bit rows past 4096 packs: two reads (1024 threads of 8 packs spill: bf16
+  // [500, 40001] 71 us against 50 element by element and 34 in two reads)
+  if (!(RAG && sizeof(T) == 2 && npack > 4096) && pick_row_config(npack, l)) return;
+  if constexpr (sizeof(T) == 2 && VEC == 8 && !RAG) {
     if (npack <= (int64_t)kBwdRowItems * kBwdRowBlock) {
       EG_LAUNCH((softmax_bwd_lds<T, kBwdRowItems, kBwdRowLds, kBwdRowBlock>), dim3((unsigned)rows),
                 dim3(kBwdRowBlock), 0, st, y, dy, dx, cols);
       return;
     }
   }
-  EG_LAUNCH((softmax_bwd_loop<T, VEC, 1024, VEC * sizeof(T) == 16>), dim3((unsigned)rows),
+  EG_LAUNCH((softmax_bwd_loop<T, VEC, 1024, VEC * sizeof(T) == 16, RAG>), dim3((unsigned)rows),
             dim3(1024), 0, st, y, dy, dx, cols);
+}
+
+// Rows that are not whole aligned packs: unaligned 16-byte packs (bf16 [2000, 10007]
+// forward and backward 91.2 -> 49.6 us, fp32 [8000, 1001] 38.2 -> 31.3, [1000, 9001] 44.7 ->
+// 37.2), except fp32 rows of 4097-8192 columns, which one register row of single elements
+// takes at whole cache lines per wave ([2000, 5001] 37.9 us against 39.5, [2000, 8001] 57.2
+// against 64.4), and rows narrower than a pack.
+template <typename T>
+bool ragged_packs(int64_t cols) {
+  return cols >= (int64_t)(16 / sizeof(T)) && !(sizeof(T) == 4 && cols > 4096 && cols <= 8192);
 }
 
 int check_dims(const char* what, int64_t rows, int64_t cols) {
@@ -521,6 +534,8 @@ extern "C" int eg_softmax_fwd(const void* x, void* y, int64_t rows, int64_t cols
     T* yp = static_cast<T*>(y);
     if (cols % V == 0 && aligned16(x) && aligned16(y))
       softmax_fwd_vec<T, V>(xp, yp, rows, (int)cols, st);
+    else if (ragged_packs<T>(cols))
+      softmax_fwd_vec<T, V, true>(xp, yp, rows, (int)cols, st);
     else
       softmax_fwd_vec<T, 1>(xp, yp, rows, (int)cols, st);
     return check_launch("eg_softmax_fwd");
@@ -542,6 +557,8 @@ extern "C" int eg_softmax_bwd(const void* y, const void* dy, void* dx, int64_t r
     T* dp = static_cast<T*>(dx);
     if (cols % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx))
       softmax_bwd_vec<T, V>(yp, gp, dp, rows, (int)cols, st);
+    else if (ragged_packs<T>(cols))
+      softmax_bwd_vec<T, V, true>(yp, gp, dp, rows, (int)cols, st);
     else
       softmax_bwd_vec<T, 1>(yp, gp, dp, rows, (int)cols, st);
     return check_launch("eg_softmax_bwd");

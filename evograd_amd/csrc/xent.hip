@@ -19,10 +19,12 @@
 //                     thread 0) into the workspace.
 //   xent_mean_kernel  one workgroup: the row losses summed in a fixed order and
 //                     the non-ignored rows counted; writes the loss and n_valid.
-//   xent_bwd_flat_kernel  wide rows: one read of the logits and one write of
-//                     dlogits, workgroups in address order over the flattened
-//                     matrix; dloss read from device memory.
-//   xent_bwd_rows_kernel  narrow rows: one workgroup per row.
+//   xent_bwd_flat_kernel  one read of the logits and one write of dlogits, workgroups
+//                     in address order over the flattened matrix; dloss read from
+//                     device memory.
+// Rows that are no multiple of a 16-byte pack are read and written in unaligned packs
+// (eg_common.hpp): bf16 [4096, 50257] forward and backward 677 us element by element, 229
+// so; fp32 backward 1.5x faster at any odd width past 2500.
 //   scale_copy_kernel dst = src * mul / div with a dtype conversion (the fused
 //                     linear cross entropy's dweight conversion and its dloss / n
 //                     scaling).
@@ -47,10 +49,9 @@ using rowwise::kFlatUnroll;
 using rowwise::kLog2e;
 using rowwise::kUnroll;
 using rowwise::pick_row_block;
-constexpr int kBwdBlock = 256;
 constexpr int kMeanBlock = 1024;
 
-template <typename T, int VEC, int BLOCK, bool NT>
+template <typename T, int VEC, int BLOCK, bool NT, bool RAG>
 __global__ __launch_bounds__(BLOCK) void xent_lse_kernel(const T* __restrict__ x,
                                                          const int64_t* __restrict__ target,
                                                          float* __restrict__ lse,
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(BLOCK) void xent_lse_kernel(const T* __restrict__ x
     t = target[row];
     if (t != ignore_index) picked = (t >= 0 && t < cols) ? to_f32(xr[t]) : NAN;
   }
-  const float l = rowwise::row_lse<T, VEC, BLOCK, NT>(xr, cols, red);
+  const float l = rowwise::row_lse<T, VEC, BLOCK, NT, RAG>(xr, cols, red);
   if (threadIdx.x == 0) {
     lse[row] = l;
     rowloss[row] = (t == ignore_index) ? 0.f : l - picked;
@@ -154,69 +155,61 @@ __device__ __forceinline__ void grad_pack(const RowGrad& rg, int c, const float 
   }
 }
 
-// Wide rows: the matrix as one flat sequence of packs, workgroup b covering
-// packs [b * kFlatPer, (b + 1) * kFlatPer) in address order, so the workgroups in
-// flight stream through contiguous memory. A workgroup spans at most two rows
-// (packs per row >= kFlatPer, checked by the host). TI is the logits type, TO the
-// gradient's, TD the type of dloss.
-template <typename TI, typename TO, typename TD, int VEC, bool NT>
+// The matrix as one flat sequence of packs, workgroup b covering packs [b * kFlatPer,
+// (b + 1) * kFlatPer) in address order, so the workgroups in flight stream through
+// contiguous memory. With at least kFlatPer packs per row a workgroup spans at most two
+// rows, whose factors every thread holds; with narrower rows (MANY) each pack finds its
+// row by a 32-bit division and takes that row's factors (one workgroup per row instead
+// left most of its threads without a pack: bf16
+// [8000, 1000] 10.3 -> 8.8 us, fp32 [8000, 501] 8.7 -> 7.8).
+// RAG: ragged rows. TI is the logits type, TO the gradient's, TD the type of dloss.
+template <typename TI, typename TO, typename TD, int VEC, bool NT, bool RAG, bool MANY>
 __global__ __launch_bounds__(kFlatBlock) void xent_bwd_flat_kernel(
     const TD* __restrict__ dloss, const TI* __restrict__ x, const int64_t* __restrict__ target,
     const float* __restrict__ lse, const float* __restrict__ n_valid, TO* __restrict__ dx,
     int64_t rows, int cols, int64_t ldd, int64_t ignore_index) {
-  const int64_t ppr = cols / VEC;  // packs per row
+  const int64_t ppr = (cols + VEC - 1) / VEC;  // packs per row
   const int64_t npack = rows * ppr;
   const int64_t first = (int64_t)blockIdx.x * kFlatPer;
   const int64_t row0 = first / ppr;
-  const int64_t bound = (row0 + 1) * ppr;  // first pack of the next row
-  const RowGrad r0 = row_grad(dloss, target, lse, n_valid, row0, cols, ignore_index);
-  const bool two = first + kFlatPer > bound && row0 + 1 < rows;
-  const RowGrad r1 = two ? row_grad(dloss, target, lse, n_valid, row0 + 1, cols, ignore_index)
-                         : r0;
+  const int64_t at0 = row0 * ppr;
+  RowGrad rg[MANY ? kFlatUnroll : 2];
+  if constexpr (!MANY) {
+    rg[0] = row_grad(dloss, target, lse, n_valid, row0, cols, ignore_index);
+    const bool two = first + kFlatPer > at0 + ppr && row0 + 1 < rows;
+    rg[1] = two ? row_grad(dloss, target, lse, n_valid, row0 + 1, cols, ignore_index) : rg[0];
+  }
+  // row of this thread's pack u, counted from row0, and the pack
+  auto at = [&](int u, int& r) {
+    const unsigned q = (unsigned)(first - at0) + u * kFlatBlock + threadIdx.x;
+    r = MANY ? (int)(q / (unsigned)ppr) : q >= (unsigned)ppr ? 1 : 0;
+    const int c = (int)(q - (unsigned)r * (unsigned)ppr) * VEC;
+    return RAG ? ragged_pack<VEC>(c, cols) : RaggedPack{c, 0};
+  };
   float v[kFlatUnroll][VEC];
 #pragma unroll
   for (int u = 0; u < kFlatUnroll; ++u) {
     const int64_t p = first + u * kFlatBlock + threadIdx.x;
-    if (p < npack) load_vec<TI, VEC, NT>(x + p * VEC, v[u]);
+    if (p < npack) {
+      int r;
+      const RaggedPack k = at(u, r);
+      if constexpr (RAG) load_ragged<TI, VEC, NT>(x + (row0 + r) * cols + k.c, v[u]);
+      else load_vec<TI, VEC, NT>(x + p * VEC, v[u]);
+      if constexpr (MANY)
+        rg[u] = row_grad(dloss, target, lse, n_valid, row0 + r, cols, ignore_index);
+    }
   }
 #pragma unroll
   for (int u = 0; u < kFlatUnroll; ++u) {
-    const int64_t p = first + u * kFlatBlock + threadIdx.x;
-    if (p < npack) {
-      const bool hi = p >= bound;
-      const int c = (int)((hi ? p - bound : p - row0 * ppr) * VEC);
+    if (first + u * kFlatBlock + threadIdx.x < npack) {
+      int r;
+      const RaggedPack k = at(u, r);
       float o[VEC];
-      grad_pack<VEC>(hi ? r1 : r0, c, v[u], o);
-      store_vec<TO, VEC, NT>(dx + (row0 + (hi ? 1 : 0)) * ldd + c, o);
-    }
-  }
-}
-
-// Narrow rows (fewer packs than one flat workgroup covers): one workgroup per row.
-template <typename TI, typename TO, typename TD, int VEC, bool NT>
-__global__ __launch_bounds__(kBwdBlock) void xent_bwd_rows_kernel(
-    const TD* __restrict__ dloss, const TI* __restrict__ x, const int64_t* __restrict__ target,
-    const float* __restrict__ lse, const float* __restrict__ n_valid, TO* __restrict__ dx,
-    int cols, int64_t ldd, int64_t ignore_index) {
-  constexpr int STEP = kBwdBlock * VEC;
-  const int64_t row = blockIdx.x;
-  const RowGrad rg = row_grad(dloss, target, lse, n_valid, row, cols, ignore_index);
-  const int c0 = (int)blockIdx.y * (STEP * kUnroll) + (int)threadIdx.x * VEC;
-  const TI* __restrict__ xr = x + row * cols;
-  TO* __restrict__ dr = dx + row * ldd;
-  float v[kUnroll][VEC];
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int c = c0 + u * STEP;
-    if (c < cols && !rg.ignored) load_vec<TI, VEC, NT>(xr + c, v[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int c = c0 + u * STEP;
-    if (c < cols) {
-      float o[VEC];
-      grad_pack<VEC>(rg, c, v[u], o);
-      store_vec<TO, VEC, NT>(dr + c, o);
+      if constexpr (MANY) grad_pack<VEC>(rg[u], k.c, v[u], o);
+      else grad_pack<VEC>(r ? rg[1] : rg[0], k.c, v[u], o);
+      TO* d = dx + (row0 + r) * ldd + k.c;
+      if constexpr (RAG) store_ragged<TO, VEC, NT>(d, k.lo, o);
+      else store_vec<TO, VEC, NT>(d, o);
     }
   }
 }
@@ -253,34 +246,31 @@ __global__ __launch_bounds__(256) void scale_copy_kernel(const TS* __restrict__ 
   }
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG = false>
 struct LseLaunch {
   const T* x; const int64_t* target; float* lse; float* rowloss; int64_t rows; int cols;
   int64_t ignore_index; hipStream_t st;
   template <int BLOCK> void go() {
-    EG_LAUNCH((xent_lse_kernel<T, VEC, BLOCK, VEC * sizeof(T) == 16>), dim3((unsigned)rows),
+    EG_LAUNCH((xent_lse_kernel<T, VEC, BLOCK, VEC * sizeof(T) == 16, RAG>), dim3((unsigned)rows),
               dim3(BLOCK), 0, st, x, target, lse, rowloss, cols, ignore_index);
   }
 };
 
-template <typename TI, typename TO, typename TD, int VEC>
-// dlogits rows are written with row stride ldd (>= cols, a multiple of VEC).
+// dlogits rows are written with row stride ldd (>= cols, a multiple of VEC unless RAG).
+template <typename TI, typename TO, typename TD, int VEC, bool RAG = false>
 void launch_bwd(const TD* gp, const TI* xp, const int64_t* target, const float* lse,
                 const float* n_valid, TO* dp, int64_t rows, int cols, int64_t ignore_index,
                 hipStream_t st, int64_t ldd = -1) {
   constexpr bool NT = VEC * sizeof(TI) == 16;
   if (ldd < 0) ldd = cols;
-  const int64_t ppr = cols / VEC;
-  if (ppr >= kFlatPer) {
-    const int64_t blocks = (rows * ppr + kFlatPer - 1) / kFlatPer;
-    EG_LAUNCH((xent_bwd_flat_kernel<TI, TO, TD, VEC, NT>), dim3((unsigned)blocks),
-              dim3(kFlatBlock), 0, st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd,
-              ignore_index);
-  } else {
-    EG_LAUNCH((xent_bwd_rows_kernel<TI, TO, TD, VEC, NT>), dim3((unsigned)rows, 1u),
-              dim3(kBwdBlock), 0, st, gp, xp, target, lse, n_valid, dp, cols, ldd,
-              ignore_index);
-  }
+  const int64_t ppr = (cols + VEC - 1) / VEC;
+  const dim3 grid((unsigned)((rows * ppr + kFlatPer - 1) / kFlatPer));
+  if (ppr >= kFlatPer)
+    EG_LAUNCH((xent_bwd_flat_kernel<TI, TO, TD, VEC, NT, RAG, false>), grid, dim3(kFlatBlock), 0,
+              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index);
+  else
+    EG_LAUNCH((xent_bwd_flat_kernel<TI, TO, TD, VEC, NT, RAG, true>), grid, dim3(kFlatBlock), 0,
+              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index);
 }
 
 int check_xent(const char* what, int64_t rows, int64_t cols) {
@@ -330,6 +320,9 @@ extern "C" int eg_cross_entropy_fwd(const void* logits, const int64_t* target, v
       if (cols % V == 0 && aligned16(logits)) {
         pick_row_block(cols / V, LseLaunch<T, V>{xp, target, lse, rowloss, rows, (int)cols,
                                                  ignore_index, st});
+      } else if (cols >= V) {
+        pick_row_block((cols + V - 1) / V, LseLaunch<T, V, true>{xp, target, lse, rowloss, rows,
+                                                                 (int)cols, ignore_index, st});
       } else {
         pick_row_block(cols, LseLaunch<T, 1>{xp, target, lse, rowloss, rows, (int)cols,
                                              ignore_index, st});
@@ -370,6 +363,9 @@ extern "C" int eg_cross_entropy_bwd(const void* dloss, const void* logits,
     if (cols % V == 0 && aligned16(logits) && aligned16(dlogits))
       launch_bwd<T, T, T, V>(gp, xp, target, lse, n_valid, dp, rows, (int)cols, ignore_index,
                              st);
+    else if (cols >= V)
+      launch_bwd<T, T, T, V, true>(gp, xp, target, lse, n_valid, dp, rows, (int)cols,
+                                   ignore_index, st);
     else
       launch_bwd<T, T, T, 1>(gp, xp, target, lse, n_valid, dp, rows, (int)cols, ignore_index,
                              st);
@@ -388,7 +384,7 @@ extern "C" int eg_cross_entropy_bwd(const void* dloss, const void* logits,
 //   losses and unit dlogits = softmax - onehot in place (one chunk of all rows by
 //   default: no fp32 logits are held);
 //   fp32 inputs: logits = x_c W^T (fp32) -> lse and row losses (xent_lse_kernel)
-//   -> unit dlogits (xent_bwd_*_kernel), chunks of at most 2^29 logits;
+//   -> unit dlogits (xent_bwd_flat_kernel), chunks of at most 2^29 logits;
 // then dx_c = dl_c W and dW (+)= dl_c^T x_c (MFMA; with more than one chunk the
 // products accumulate in an fp32 [vocab, hidden] buffer, added in each product's
 // epilogue, and the last chunk's product rounds the sum once into dW; fp32 inputs
@@ -763,6 +759,12 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
                                                         ignore_index, st});
           launch_bwd<float, T, float, 4>(none, logits, target + r0, lse + r0, nullptr, dlp, n,
                                          (int)vocab, ignore_index, st, L.vp);
+        } else if (vocab >= 4) {
+          pick_row_block((vocab + 3) / 4, LseLaunch<float, 4, true>{logits, target + r0, lse + r0,
+                                                                    rowloss + r0, n, (int)vocab,
+                                                                    ignore_index, st});
+          launch_bwd<float, T, float, 4, true>(none, logits, target + r0, lse + r0, nullptr, dlp,
+                                               n, (int)vocab, ignore_index, st, L.vp);
         } else {
           pick_row_block(vocab, LseLaunch<float, 1>{logits, target + r0, lse + r0, rowloss + r0,
                                                     n, (int)vocab, ignore_index, st});
