@@ -71,25 +71,25 @@ namespace {
 int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
               int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
               int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
-              const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes,
+              const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int fixed_splits,
               const SegArgs& seg);
 }  // namespace
 
 int gemm_launch(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                 int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
                 int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
-                const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes) {
+                const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int splits) {
   SegArgs none{};
   none.dim = kSegNone;
   return gemm_impl(A, B, C, M, N, K, lda, ldb, ldc, a_kc, b_kc, a_rows, b_rows, dtype, c_dtype, st,
-                   name, R, ldr, r_f32, ws, ws_bytes, none);
+                   name, R, ldr, r_f32, ws, ws_bytes, splits, none);
 }
 
 namespace {
 int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
               int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
               int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
-              const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes,
+              const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int fixed_splits,
               const SegArgs& seg) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0) {
@@ -172,11 +172,13 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
   // 16-byte aligned base; otherwise the kernel stores element by element.
   const int vec_c = (ldc % 4 == 0) && aligned16(C) &&
                     (!R || ((ldr % 4 == 0) && aligned16(R)));
-  const bool ws_ok = ws && aligned16(ws) && ws_bytes >= gemm_workspace_bytes(M, N, K);
-  int splits = gemm_splits(M, N, K);
+  const size_t need = fixed_splits > 0 ? (size_t)fixed_splits * M * N * sizeof(float)
+                                       : gemm_workspace_bytes(M, N, K);
+  const bool ws_ok = ws && aligned16(ws) && ws_bytes >= need;
+  int splits = fixed_splits > 0 ? fixed_splits : gemm_splits(M, N, K);
   if (splits > 1 && !ws_ok) splits = 1;
   TailPlan tp = gemm_tail(M, N, K);
-  if (!ws_ok) tp = TailPlan{tiles, 0, 1, 0};
+  if (!ws_ok || fixed_splits > 0) tp = TailPlan{tiles, 0, 1, 0};
   const int nk = (int)((K + kBK - 1) / kBK);
   const int kt_per = tp.tail ? tp.kt_per : (nk + splits - 1) / splits;
   const unsigned grid_x = tp.tail ? (unsigned)(tp.head + tp.tail * tp.parts) : grid;
@@ -398,5 +400,5 @@ extern "C" int eg_gemm_segmented(const void* a, const void* b, void* c, int64_t 
   if (m == 0 || n == 0) return 0;
   return gemm_impl(pa, pb, pc, m, n, k, lda, ldb, ldc, akc, bkc, akc ? m : k, bkc ? n : k, dtype,
                    c_dtype, as_stream(stream), name, nullptr, 0, false, workspace,
-                   workspace_bytes, g);
+                   workspace_bytes, 0, g);
 }
