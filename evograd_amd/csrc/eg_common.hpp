@@ -295,8 +295,8 @@ int zero_fill(void* p, size_t bytes, hipStream_t st, const char* what);
 // accumulates in place. With a workspace of at least gemm_workspace_bytes(m, n, k)
 // a product of few output tiles splits k (fp32 partials, a fixed-order sum). splits > 0
 // fixes the k ranges of a 16-bit product whatever its row count (1: none; workspace
-// splits x m x n x 4 bytes); gemm_splits is the choice for a shape.
-int gemm_splits(int64_t m, int64_t n, int64_t k);
+// splits x m x n x 4 bytes); gemm_plan_splits is the choice for a shape.
+int gemm_plan_splits(int64_t m, int64_t n, int64_t k);
 size_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int gemm_launch(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k,
                 int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,

@@ -2,12 +2,15 @@
 // cross entropy's logits product): shape checks, split-K and split-tail planning,
 // launches. The kernels are in gemm_kernel.hpp, instantiated by gemm_inst_*.hip.
 #include "gemm_kernel.hpp"
+#include "gemm_mid.hpp"
 
 namespace eg {
 namespace gk {
 // The product kernels are instantiated in the gemm_inst_*.hip sources, not here.
 EG_GEMM_ALL_KERNELS(extern template, bf16_t)
 EG_GEMM_ALL_KERNELS(extern template, f16_t)
+EG_MID_ALL_KERNELS(extern template, bf16_t)
+EG_MID_ALL_KERNELS(extern template, f16_t)
 }  // namespace gk
 using namespace gk;
 
@@ -26,6 +29,48 @@ int gemm_splits(int64_t M, int64_t N, int64_t K) {
   if (s < 2) return 1;
   const int64_t per = (nk + s - 1) / s;
   return (int)((nk + per - 1) / per);
+}
+
+// Which kernel a product of at most kSplitTarget / 2 tiles of 256 x 256 runs on, and its
+// split of k: the cheaper of the two by a cost in us fitted to both kernels over outputs
+// of 77-2048 x 256-28672 at depths 77-28672 (bf16, three layouts; within 15% of most).
+// A 256 x 256 workgroup costs 10 + 1.63 per 64-deep slice, a 128 x 128 one 5 + 0.62; 256
+// run at a time; a split adds its reduction, 8 + the partials at 5 TB/s. So the 128 x 128
+// kernel takes small outputs and short depths (77 x 256 x 256: 13.6 -> 6.8 us, 600 x 3584 x
+// 1024: 28.9 -> 15.2, 2048 x 2048 x 1024: 37.0 -> 16.1, 1024 x 4096 x 4096: 54.6 -> 42.9) and
+// the 256 x 256 one long depths (1024 x 4096 x 14336: 123 against 166) and every larger
+// output (2048 x 7168 x 1024, 224 tiles: 36 against 54).
+// The 128 x 128 kernel never takes more parts than gemm_splits, whose partials the
+// caller's workspace is sized for.
+struct GemmPlan {
+  bool mid;
+  int splits;
+};
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int max_splits, int fixed_splits) {
+  auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
+  const int64_t nk = (K + kBK - 1) / kBK, big = tiles(kBM), small = tiles(kMT);
+  auto cost = [&](int64_t t, double fixed, double slice, int64_t s) {
+    const int64_t waves = (t * s + kSplitTarget - 1) / kSplitTarget;
+    const double run = (double)waves * (fixed + slice * (double)((nk + s - 1) / s));
+    return s > 1 ? run + 8.0 + (double)s * (double)M * (double)N * 4e-6 / 5.0 : run;
+  };
+  const int sb = fixed_splits > 0 ? fixed_splits : std::min(max_splits, gemm_splits(M, N, K));
+  GemmPlan best{false, sb};
+  if (big > kSplitTarget / 2) return best;
+  double least = cost(big, 10.0, 1.63, sb);
+  for (int s = fixed_splits > 0 ? fixed_splits : 1; s <= sb; ++s) {
+    if (fixed_splits <= 0 && s > 1 && small * s > kSplitTarget) break;
+    const double c = cost(small, 5.0, 0.62, s);
+    if (c < least) {
+      const int64_t per = (nk + s - 1) / s;
+      least = c;
+      best = GemmPlan{true, fixed_splits > 0 ? s : (int)((nk + per - 1) / per)};
+    }
+  }
+  return best;
+}
+int gemm_plan_splits(int64_t M, int64_t N, int64_t K) {
+  return gemm_plan(M, N, K, kMaxSplits, 0).splits;
 }
 
 // Split tail: a product of more than one wave of tiles (kSplitTarget workgroups per
@@ -175,10 +220,13 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
   const size_t need = fixed_splits > 0 ? (size_t)fixed_splits * M * N * sizeof(float)
                                        : gemm_workspace_bytes(M, N, K);
   const bool ws_ok = ws && aligned16(ws) && ws_bytes >= need;
-  int splits = fixed_splits > 0 ? fixed_splits : gemm_splits(M, N, K);
-  if (splits > 1 && !ws_ok) splits = 1;
+  const GemmPlan plan = gemm_plan(M, N, K, ws_ok ? kMaxSplits : 1, ws_ok ? fixed_splits : 0);
+  const bool mid = plan.mid;
+  const int splits = plan.splits;
   TailPlan tp = gemm_tail(M, N, K);
-  if (!ws_ok || fixed_splits > 0) tp = TailPlan{tiles, 0, 1, 0};
+  if (!ws_ok || fixed_splits > 0 || mid) tp = TailPlan{tiles, 0, 1, 0};
+  const int64_t mid_m = (M + kMT - 1) / kMT, mid_tiles = mid_m * ((N + kMT - 1) / kMT);
+  const dim3 mid_grid((unsigned)((mid_tiles + 7) / 8 * 8), (unsigned)splits);
   const int nk = (int)((K + kBK - 1) / kBK);
   const int kt_per = tp.tail ? tp.kt_per : (nk + splits - 1) / splits;
   const unsigned grid_x = tp.tail ? (unsigned)(tp.head + tp.tail * tp.parts) : grid;
@@ -187,7 +235,23 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
     using TC = decltype(ctag);
     constexpr bool AK = decltype(akc)::value, BK = decltype(bkc)::value;
     float* part = (splits > 1 || tp.tail) ? (float*)ws : nullptr;
-    if (seg.dim != kSegNone) {
+    if (mid) {
+      auto run = [&](auto segc) {
+        EG_LAUNCH((gemm_mid_kernel<T, AK, BK, TC, decltype(segc)::value>), mid_grid, dim3(256), 0,
+                  st, (const uint16_t*)A, (const uint16_t*)B, (TC*)C, (int)M, (int)N, (int)K, lda,
+                  ldb, ldc, a_rows, b_rows, (int)mid_m, (int)mid_tiles, vec_c, R, ldr, (int)r_f32,
+                  kt_per, part, seg);
+      };
+      if (seg.dim == kSegNone) {
+        run(std::integral_constant<int, 0>{});
+      } else if constexpr (std::is_same<T, TC>::value) {
+        if (seg.dim == kSegK) run(std::integral_constant<int, 2>{});
+        else run(std::integral_constant<int, 1>{});
+      } else {
+        set_error("%s: segmented products write C in the operands' dtype", name);
+        return 1;
+      }
+    } else if (seg.dim != kSegNone) {
       // segmented products: 16-bit C only (one more instantiation per layout)
       if constexpr (std::is_same<T, TC>::value) {
         if (seg.dim == kSegK)

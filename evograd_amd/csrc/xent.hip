@@ -718,7 +718,7 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
   int dx_splits = 0;
   if (dtype != EG_F32) {
     const int64_t fit = (int64_t)(dw_bytes / ((size_t)rows * hidden * sizeof(float)));
-    const int64_t nk = L.vp / 64, s = std::min<int64_t>(fit, gemm_splits(rows, hidden, L.vp));
+    const int64_t nk = L.vp / 64, s = std::min<int64_t>(fit, gemm_plan_splits(rows, hidden, L.vp));
     const int64_t per = s > 1 ? (nk + s - 1) / s : nk;
     dx_splits = (int)((nk + per - 1) / per);
   }

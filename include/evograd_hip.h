@@ -373,8 +373,8 @@ int eg_scale_copy(const void* src, int src_dtype, void* dst, int dst_dtype, int6
  * 16-byte aligned.
  * Products with at most half as many output tiles (256 x 256) as an MI355X has CUs
  * split k over workgroups when `workspace` holds at least
- * eg_gemm_workspace_bytes(m, n, k, dtype) bytes (else, or with workspace NULL, they
- * run unsplit): each k range writes an fp32 partial, and a second pass sums them in
+ * eg_gemm_workspace_bytes(m, n, k, dtype) bytes and splitting is the faster choice for
+ * the shape (else, or with workspace NULL, they run unsplit): each k range writes an fp32 partial, and a second pass sums them in
  * a fixed order, adds r and rounds c once. So do the tiles of a last wave that is at
  * most half full (more than 256 tiles), and fp32 products of fewer than 256 tiles of
  * 32 x 32 (at most 8 ranges). The split depends on the shape only, so results are bitwise repeatable. */
