@@ -155,7 +155,7 @@ __device__ __forceinline__ RaggedPack ragged_pack(int c, int cols) {
 }
 // NT: with the non-temporal hint (16-byte packs only, as in load_vec).
 template <typename T, int VEC, bool NT>
-__device__ __forceinline__ void load_ragged(const T* __restrict__ p, float (&out)[VEC]) {
+__device__ __forceinline__ Pack<T, VEC> load_ragged_raw(const T* __restrict__ p) {
   typedef unsigned int words __attribute__((ext_vector_type(sizeof(T) * VEC / 4)));
   typedef words __attribute__((aligned(sizeof(T)))) any_words;
   const any_words* a = reinterpret_cast<const any_words*>(p);
@@ -164,6 +164,11 @@ __device__ __forceinline__ void load_ragged(const T* __restrict__ p, float (&out
   else raw = *a;
   Pack<T, VEC> pk;
   __builtin_memcpy(&pk, &raw, sizeof(raw));
+  return pk;
+}
+template <typename T, int VEC, bool NT>
+__device__ __forceinline__ void load_ragged(const T* __restrict__ p, float (&out)[VEC]) {
+  const Pack<T, VEC> pk = load_ragged_raw<T, VEC, NT>(p);
 #pragma unroll
   for (int i = 0; i < VEC; ++i) out[i] = to_f32(pk.v[i]);
 }

@@ -38,6 +38,7 @@
 // workgroup per row.
 #include "eg_common.hpp"
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 
@@ -63,6 +64,24 @@ constexpr int64_t bwd_per512(bool ln, bool add) {
 inline int64_t ring_blocks(int64_t rows, int64_t per512, int block) {
   const int64_t g = per512 * (block < 512 ? 512 / block : 1);
   return rows < g ? (rows > 0 ? rows : 1) : g;
+}
+
+// Workgroups of a one-stream backward ring: every one of them writes a partial row that
+// the column sum reads back, so a ring narrower than 512 threads takes 256 x 512 / block of
+// them at most, and fewer, down to 512, while each would walk under 8 rows (with 512 x
+// 512 / block, a workgroup of bf16 [4000, 512] wrote one fp32 partial row per 16-bit row
+// it read). Backward call, bf16, before and after: RMSNorm [4000, 512] 17.7 -> 10.5 us,
+// [8000, 1024] 21.2 -> 16.4, [16000, 512] 25.0 -> 17.7, [16000, 2048] 41.7 -> 38.0;
+// LayerNorm [4000, 1024] 21.3 -> 13.8, [65536, 512] 52.1 -> 44.0; 256 workgroups, or 4096
+// at 64 threads, are slower at each of these. fp32 rings of 256 threads keep the larger
+// count below 2048 rows ([1500, 1000]: 12.6 us against 10.6): the declared fp32 gate, 1e-5
+// against an fp32 oracle that is itself up to 1.2 times that off 64 bits at such sizes,
+// has no room there for another order of the same sums.
+inline int64_t bwd_ring_blocks(int64_t rows, int64_t per512, int block, int elem) {
+  if (block >= 512 || (block == 256 && elem == 4 && rows < 2048))
+    return ring_blocks(rows, per512, block);
+  const int64_t g = std::min<int64_t>(256 * 512 / block, std::max<int64_t>(512, rows / 8));
+  return std::max<int64_t>(1, std::min(rows, g));
 }
 
 // Backward rings whose row stream is one 512-thread range (rows of 257-512 packs,
@@ -721,49 +740,47 @@ __global__ __launch_bounds__(BLOCK) void norm_bwd_ring(
 }
 
 // ------------------------------------------------- stage 2: column sums
-// out[c] = sum_{g=0..G-1} partial[g][c]. A wave owns 4 adjacent columns; lane l
-// adds the partial rows l, l + 64, l + 128, ... in ascending order (batches of 8
-// loads issued together), then the 64 lane totals are combined by a butterfly.
-// The order is fixed, so the result is bit-identical on every run.
+// out[c] = sum_{g=0..G-1} partial[g][c], in a fixed order (bit-identical on every run).
 // blockIdx.y selects the parameter (0: p0 -> o0, 1: p1 -> o1).
+//
+// Any row width (colsum_wide_kernel below takes those divisible by 4): 32 adjacent columns
+// per workgroup, lane = column, 32 row groups; group k adds the partial rows k, k + 32, ...
+// (8 loads in flight, each 128 contiguous bytes per half wave, added pairwise), then the
+// groups are added pairwise. Backward call fp32 [1000, 255] 24.5 -> 9.6 us, bf16
+// [4000, 1301] 23.5 -> 15.6 (a wave per 4 columns before, its lanes a whole row apart).
 template <typename T>
-__global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p0,
-                                                     const float* __restrict__ p1,
-                                                     T* __restrict__ o0, T* __restrict__ o1,
-                                                     int G, int hidden) {
-  constexpr int kBatch = 8;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int c = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * 4;
-  if (c >= hidden) return;  // whole wave leaves together
-  const float* p = blockIdx.y == 0 ? p0 : p1;
-  T* o = blockIdx.y == 0 ? o0 : o1;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if ((hidden & 3) == 0) {
-    for (int g0 = lane; g0 < G; g0 += kWave * kBatch) {
-      float4 v[kBatch];
+__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ p0,
+                                                      const float* __restrict__ p1,
+                                                      T* __restrict__ o0, T* __restrict__ o1,
+                                                      int G, int hidden) {
+  constexpr int kCols = 32, kGroups = 1024 / kCols, kBatch = 8;
+  __shared__ float red[kGroups][kCols + 1];
+  const int cl = threadIdx.x % kCols, rg = threadIdx.x / kCols;
+  const int c = (int)blockIdx.x * kCols + cl;
+  const float* p = (blockIdx.y == 0 ? p0 : p1) + (c < hidden ? c : 0);
+  float acc = 0.f;
+  for (int g0 = rg; g0 < G; g0 += kGroups * kBatch) {
+    float v[kBatch];
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int g = g0 + kWave * i;
-        v[i] = g < G ? *reinterpret_cast<const float4*>(p + (int64_t)g * hidden + c)
-                     : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        acc[0] += v[i].x; acc[1] += v[i].y; acc[2] += v[i].z; acc[3] += v[i].w;
-      }
+    for (int i = 0; i < kBatch; ++i) {
+      const int g = g0 + kGroups * i;
+      const float y = p[(int64_t)(g < G ? g : 0) * hidden];
+      v[i] = g < G ? y : 0.f;
     }
-  } else {
-    for (int g = lane; g < G; g += kWave)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c + i < hidden) acc[i] += p[(int64_t)g * hidden + c + i];
+    acc += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
+  red[rg][cl] = acc;
+  __syncthreads();
+  if (rg == 0 && c < hidden) {
+    float s[kGroups];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = wave_reduce(acc[i], SumOp());
-  if (lane == 0)
+    for (int k = 0; k < kGroups; ++k) s[k] = red[k][cl];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (c + i < hidden) o[c + i] = from_f32<T>(acc[i]);
+    for (int w = kGroups / 2; w >= 1; w >>= 1)
+#pragma unroll
+      for (int k = 0; k < w; ++k) s[k] += s[k + w];
+    (blockIdx.y == 0 ? o0 : o1)[c] = from_f32<T>(s[0]);
+  }
 }
 
 // Column sums of G partial rows when hidden % 4 == 0: a 1024-thread workgroup per
@@ -841,8 +858,8 @@ int launch_colsum(const float* p0, const float* p1, T* o0, T* o1, int nparams, i
               dim3((unsigned)((quads + kColsumQuads - 1) / kColsumQuads), (unsigned)nparams),
               dim3(1024), 0, st, p0, p1, o0, o1, G, hidden);
   } else {
-    EG_LAUNCH((colsum_kernel<T>), dim3((unsigned)((quads + 3) / 4), (unsigned)nparams),
-              dim3(256), 0, st, p0, p1, o0, o1, G, hidden);
+    EG_LAUNCH((colsum_kernel<T>), dim3((unsigned)((hidden + 31) / 32), (unsigned)nparams),
+              dim3(1024), 0, st, p0, p1, o0, o1, G, hidden);
   }
   return check_launch(what);
 }
@@ -875,7 +892,7 @@ struct BwdRing {
                 0, st, dy, x, res, w, mean, rstd, dx, pw, pb, rows, hidden);
       return true;
     }
-    const int64_t G = ring_blocks(rows, bwd_per512(LN, ADD), BLOCK);
+    const int64_t G = bwd_ring_blocks(rows, bwd_per512(LN, ADD), BLOCK, sizeof(T));
     EG_LAUNCH((norm_bwd_ring<T, VEC, ITEMS, BLOCK, D, LN, ADD>), dim3((unsigned)G), dim3(BLOCK),
               0, st, dy, x, res, w, mean, rstd, dx, pw, pb, rows, hidden);
     return true;
@@ -895,6 +912,7 @@ int check_norm_dims(const char* what, int64_t rows, int64_t hidden) {
   return 0;
 }
 
+
 template <typename T>
 bool vec_ok(int hidden, std::initializer_list<const void*> ptrs) {
   constexpr int V = 16 / sizeof(T);
@@ -904,8 +922,220 @@ bool vec_ok(int hidden, std::initializer_list<const void*> ptrs) {
   return true;
 }
 
-// Partial rows of the backward for a given dtype width (must match the launch).
+// ------------------------------------------- small-shape backward, one launch
+// For few rows (the reference's small regime, under 4096 tokens) the ring backward
+// and its column sum are two latency-bound launches: at bf16 [1024, 4096] 10.2 and
+// 4.0 us, for 25 MB. This kernel does the whole backward in one launch with no
+// partial rows, in two kinds of workgroups:
+//   column workgroups (first): 4 packs of columns each, 64 row lanes; lane walks
+//     rows rl, rl + 64, ... (8 rows' loads in flight) summing dy * xhat (and dy) per
+//     column in fp32 (compensated), then the 64 lane sums are added in a fixed
+//     pairwise tree ->
+//     dweight (dbias): bitwise repeatable, and read from dy, x and the saved row
+//     statistics alone;
+//   row workgroups: one row each, two passes over the row (the second from L2):
+//     the row sums, then dx.
+// dy and x are read twice (once per role), which at these sizes the 256 MB
+// Infinity Cache serves; for wide batches the ring, which reads them once, is
+// the program to use. ADD: the normalised row is x + res.
+constexpr int kSmallBlock = 256, kSmallPacks = 4, kSmallLanes = kSmallBlock / kSmallPacks;
+constexpr int kSmallUnroll = 8;  // rows of a lane whose loads are issued together
+
+template <typename T, int VEC, bool LN, bool ADD, bool RAG>
+__global__ __launch_bounds__(kSmallBlock) void norm_bwd_small(
+    const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ res,
+    const T* __restrict__ w,
+    const float* __restrict__ mean, const float* __restrict__ rstd, T* __restrict__ dx,
+    T* __restrict__ dweight, T* __restrict__ dbias, int64_t rows, int hidden, int ncolwg) {
+  __shared__ float part[2][kSmallLanes][kSmallPacks * VEC];
+  __shared__ float red[2][kSmallBlock / kWave];
+  const int t = threadIdx.x;
+  // the pack at column c: where it is read, and its first own element
+  auto pack_at = [&](int c) { return RAG ? ragged_pack<VEC>(c, hidden) : RaggedPack{c, 0}; };
+  auto load = [&](const T* p, float (&v)[VEC]) {
+    if constexpr (RAG) load_ragged<T, VEC, false>(p, v);
+    else load_f32<T, VEC>(p, v);
+  };
+  // the normalised row's values at element offset o: x, or x + res
+  auto load_x = [&](int64_t o, float (&v)[VEC]) {
+    load(x + o, v);
+    if constexpr (ADD) {
+      float a[VEC];
+      load(res + o, a);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) v[i] += a[i];
+    }
+  };
+  if ((int)blockIdx.x < ncolwg) {
+    const int p = t % kSmallPacks, rl = t / kSmallPacks;
+    const int first = ((int)blockIdx.x * kSmallPacks + p) * VEC;
+    const bool live = first < hidden;
+    const int c0 = live ? pack_at(first).c : 0;
+    // Compensated (Kahan) sums per lane, then a pairwise tree over the 64 lanes: a
+    // lane's rows are summed in order with their rounding errors carried, so the
+    // result stays within a few units of the exact column sum even where the rows
+    // cancel (the ring's many short partial rows give the same by splitting).
+    float sw[VEC], sb[VEC], cw[VEC], cb[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) { sw[i] = 0.f; sb[i] = 0.f; cw[i] = 0.f; cb[i] = 0.f; }
+    auto kahan = [](float& s, float& c, float v) {
+      const float y = v - c;
+      const float t2 = s + y;
+      c = (t2 - s) - y;
+      s = t2;
+    };
+    if (live) {
+      // kSmallUnroll rows per batch, all their loads issued before the sums (rows
+      // past the end load row 0 and are skipped)
+      for (int64_t r0 = rl; r0 < rows; r0 += (int64_t)kSmallLanes * kSmallUnroll) {
+        float g[kSmallUnroll][VEC], xv[kSmallUnroll][VEC], rs[kSmallUnroll], mu[kSmallUnroll];
+#pragma unroll
+        for (int u = 0; u < kSmallUnroll; ++u) {
+          const int64_t r = r0 + (int64_t)u * kSmallLanes;
+          const int64_t rc = r < rows ? r : 0;
+          load(dy + rc * hidden + c0, g[u]);
+          load_x(rc * hidden + c0, xv[u]);
+          rs[u] = rstd[rc];
+          mu[u] = LN ? mean[rc] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < kSmallUnroll; ++u) {
+          if (r0 + (int64_t)u * kSmallLanes >= rows) break;
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            kahan(sw[i], cw[i], g[u][i] * ((xv[u][i] - mu[u]) * rs[u]));
+            if (LN) kahan(sb[i], cb[i], g[u][i]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      part[0][rl][p * VEC + i] = sw[i] - cw[i];
+      if (LN) part[1][rl][p * VEC + i] = sb[i] - cb[i];
+    }
+    __syncthreads();
+    if (t < kSmallPacks * VEC) {
+      // column of sum t: element t % VEC of pack t / VEC
+      const int at = ((int)blockIdx.x * kSmallPacks + t / VEC) * VEC;
+      const RaggedPack k = at < hidden ? pack_at(at) : RaggedPack{hidden, 0};
+      const int col = t % VEC >= k.lo ? k.c + t % VEC : hidden;
+      float a[kSmallLanes], b[kSmallLanes];
+#pragma unroll
+      for (int l = 0; l < kSmallLanes; ++l) {
+        a[l] = part[0][l][t];
+        b[l] = LN ? part[1][l][t] : 0.f;
+      }
+#pragma unroll
+      for (int w2 = kSmallLanes / 2; w2 >= 1; w2 >>= 1)
+#pragma unroll
+        for (int l = 0; l < w2; ++l) {
+          a[l] += a[l + w2];
+          if (LN) b[l] += b[l + w2];
+        }
+      if (col < hidden) {
+        dweight[col] = from_f32<T>(a[0]);
+        if (LN) dbias[col] = from_f32<T>(b[0]);
+      }
+    }
+    return;
+  }
+  const int64_t r = (int64_t)blockIdx.x - ncolwg;
+  const T* dyr = dy + r * hidden;
+  const float rs = rstd[r], mu = LN ? mean[r] : 0.f;
+  // pass 1: sum(g) (LayerNorm) and sum(g * xhat), g = dy * w
+  float sa = 0.f, sg = 0.f;
+  for (int c = t * VEC; c < hidden; c += kSmallBlock * VEC) {
+    const RaggedPack k = pack_at(c);
+    float g[VEC], xv[VEC], wv[VEC];
+    load(dyr + k.c, g);
+    load_x(r * hidden + k.c, xv);
+    load(w + k.c, wv);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      if (RAG && i < k.lo) continue;
+      const float gi = g[i] * wv[i];
+      sa = __builtin_fmaf(gi, (xv[i] - mu) * rs, sa);
+      if (LN) sg += gi;
+    }
+  }
+  sa = wave_reduce(sa, SumOp());
+  if (LN) sg = wave_reduce(sg, SumOp());
+  if ((t & (kWave - 1)) == 0) {
+    red[0][t / kWave] = sa;
+    red[1][t / kWave] = sg;
+  }
+  __syncthreads();
+  float ta = red[0][0], tg = red[1][0];
+#pragma unroll
+  for (int k = 1; k < kSmallBlock / kWave; ++k) {
+    ta += red[0][k];
+    tg += red[1][k];
+  }
+  const float inv_h = 1.0f / (float)hidden;
+  const float mgx = ta * inv_h, mg = LN ? tg * inv_h : 0.f;
+  // pass 2: dx = rstd * (g - mean(g) - xhat * mean(g * xhat))   (RMSNorm: no mean(g))
+  for (int c = t * VEC; c < hidden; c += kSmallBlock * VEC) {
+    const RaggedPack k = pack_at(c);
+    float g[VEC], xv[VEC], wv[VEC], o[VEC];
+    load(dyr + k.c, g);
+    load_x(r * hidden + k.c, xv);
+    load(w + k.c, wv);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const float xh = (xv[i] - mu) * rs;
+      o[i] = (g[i] * wv[i] - mg - xh * mgx) * rs;
+    }
+    if constexpr (RAG) store_ragged<T, VEC, false>(dx + r * hidden + k.c, k.lo, o);
+    else store_f32<T, VEC>(dx + r * hidden + c, o);
+  }
+}
+
+// Launches norm_bwd_small over rows > 0 (sizes and pointers already checked).
+template <typename T, bool LN, bool ADD>
+int launch_bwd_small(const T* dy, const T* x, const T* res, const T* w, const float* mean,
+                     const float* rstd, T* dx, T* dweight, T* dbias, int64_t rows, int h,
+                     hipStream_t st, const char* name) {
+  constexpr int V = 16 / sizeof(T);
+  auto go = [&](auto vc, auto rag) {
+    constexpr int VC = decltype(vc)::value;
+    const int ncol = (h + kSmallPacks * VC - 1) / (kSmallPacks * VC);
+    EG_LAUNCH((norm_bwd_small<T, VC, LN, ADD, decltype(rag)::value>),
+              dim3((unsigned)(ncol + rows)), dim3(kSmallBlock), 0, st, dy, x, res, w, mean, rstd,
+              dx, dweight, dbias, rows, h, ncol);
+    return check_launch(name);
+  };
+  if (vec_ok<T>(h, {dy, x, w, dx}) && (!ADD || aligned16(res)))
+    return go(std::integral_constant<int, V>{}, std::false_type{});
+  if (h >= V) return go(std::integral_constant<int, V>{}, std::true_type{});
+  return go(std::integral_constant<int, 1>{}, std::false_type{});
+}
+
+// The backward entry points take it up to kSmallRows rows, where one launch beats the ring
+// and its column sum at every width measured (bf16, hidden 1024 / 4096 / 8192, backward call,
+// ring against one launch: RMSNorm 64 rows 9.6 / 11.0 / 10.8 -> 6.2 / 7.2 / 9.9 us, 256 rows
+// 10.2 / 11.9 / 13.6 -> 7.1 / 8.6 / 12.8; LayerNorm 256 rows 10.4 / 13.1 / 17.2 -> 8.5 / 9.9 /
+// 12.8; narrow widths win up to about 500 rows). Its workgroups read rows that others write
+// dx for, so dx must not overlap dy, x or res; where it does the ring runs.
+constexpr int64_t kSmallRows = 256;
+bool use_bwd_small(int64_t rows, int64_t hidden, size_t elem, const void* dx,
+                   std::initializer_list<const void*> read) {
+  if (rows > kSmallRows) return false;
+  const uintptr_t n = (uintptr_t)(rows * hidden) * elem, d = (uintptr_t)dx;
+  for (const void* p : read)
+    if (p && (uintptr_t)p < d + n && d < (uintptr_t)p + n) return false;
+  return true;
+}
+
+// Partial rows of the backward (must match the launch). vec: 16-byte packs of elem-byte
+// elements, else single elements.
 int64_t bwd_blocks(int64_t rows, int64_t hidden, bool ln, bool add, bool vec, int elem) {
+  const int64_t npack = vec ? (hidden + (16 / elem) - 1) / (16 / elem) : hidden;
+  if (bwd_split(npack, add)) return split_blocks(rows, bwd_per512(ln, add));
+  return bwd_ring_blocks(rows, bwd_per512(ln, add), ring_block_for(npack), elem);
+}
+// An upper bound of it, which sizes the workspace.
+int64_t bwd_blocks_max(int64_t rows, int64_t hidden, bool ln, bool add, bool vec, int elem) {
   const int64_t npack = vec ? (hidden + (16 / elem) - 1) / (16 / elem) : hidden;
   if (bwd_split(npack, add)) return split_blocks(rows, bwd_per512(ln, add));
   return ring_blocks(rows, bwd_per512(ln, add), ring_block_for(npack));
@@ -926,7 +1156,7 @@ static size_t norm_workspace_bytes(int64_t rows, int64_t hidden, bool ln) {
     for (bool vec : {true, false}) {
       for (bool add : {false, true}) {
         if (ln && add) continue;
-        const int64_t g = bwd_blocks(rows, hidden, ln, add, vec, elem);
+        const int64_t g = bwd_blocks_max(rows, hidden, ln, add, vec, elem);
         if (g > G) G = g;
       }
     }
@@ -1012,6 +1242,10 @@ static int rms_bwd_impl(const char* name, const void* dy, const void* x, const v
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
     float* part = (float*)workspace;
+    if (use_bwd_small(rows, hidden, sizeof(T), dx, {dy, x, r}))
+      return launch_bwd_small<T, false, ADD>((const T*)dy, (const T*)x, (const T*)r,
+                                             (const T*)weight, nullptr, rstd, (T*)dx, (T*)dweight,
+                                             nullptr, rows, h, st, name);
     const bool vec = vec_ok<T>(h, {dy, x, weight, dx}) && (!ADD || aligned16(r));
     bool ok;
     if (vec) {
@@ -1124,6 +1358,10 @@ extern "C" int eg_layernorm_bwd(const void* dy, const void* x, const void* weigh
     using T = scalar_t;
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
+    if (use_bwd_small(rows, hidden, sizeof(T), dx, {dy, x}))
+      return launch_bwd_small<T, true, false>((const T*)dy, (const T*)x, (const T*)nullptr,
+                                              (const T*)weight, mean, rstd, (T*)dx, (T*)dweight,
+                                              (T*)dbias, rows, h, st, "eg_layernorm_bwd");
     const bool vec = vec_ok<T>(h, {dy, x, weight, dx});
     const int G = (int)bwd_blocks(rows, h, true, false, vec, (int)sizeof(T));
     float* pw = (float*)workspace;
@@ -1141,151 +1379,6 @@ extern "C" int eg_layernorm_bwd(const void* dy, const void* x, const void* weigh
     return launch_colsum<T>(pw, pb, (T*)dweight, (T*)dbias, 2, G, h, st,
                             "eg_layernorm_bwd(colsum)");
   });
-}
-
-// ------------------------------------------- small-shape backward, one launch
-// For few rows (the reference's small regime, under 4096 tokens) the ring backward
-// and its column sum are two latency-bound launches: at bf16 [1024, 4096] 10.2 and
-// 4.0 us, for 25 MB. This kernel does the whole backward in one launch with no
-// partial rows, in two kinds of workgroups:
-//   column workgroups (first): 4 packs of columns each, 64 row lanes; lane walks
-//     rows rl, rl + 64, ... (8 rows' loads in flight) summing dy * xhat (and dy) per
-//     column in fp32 (compensated), then the 64 lane sums are added in a fixed
-//     pairwise tree ->
-//     dweight (dbias): bitwise repeatable, and read from dy, x and the saved row
-//     statistics alone;
-//   row workgroups: one row each, two passes over the row (the second from L2):
-//     the row sums, then dx.
-// dy and x are read twice (once per role), which at these sizes the 256 MB
-// Infinity Cache serves; for wide batches the ring, which reads them once, is
-// the program to use.
-constexpr int kSmallBlock = 256, kSmallPacks = 4, kSmallLanes = kSmallBlock / kSmallPacks;
-constexpr int kSmallUnroll = 8;  // rows of a lane whose loads are issued together
-
-template <typename T, int VEC, bool LN>
-__global__ __launch_bounds__(kSmallBlock) void norm_bwd_small(
-    const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
-    const float* __restrict__ mean, const float* __restrict__ rstd, T* __restrict__ dx,
-    T* __restrict__ dweight, T* __restrict__ dbias, int64_t rows, int hidden, int ncolwg) {
-  __shared__ float part[2][kSmallLanes][kSmallPacks * VEC];
-  __shared__ float red[2][kSmallBlock / kWave];
-  const int t = threadIdx.x;
-  if ((int)blockIdx.x < ncolwg) {
-    const int p = t % kSmallPacks, rl = t / kSmallPacks;
-    const int c0 = ((int)blockIdx.x * kSmallPacks + p) * VEC;
-    const bool live = c0 < hidden;
-    // Compensated (Kahan) sums per lane, then a pairwise tree over the 64 lanes: a
-    // lane's rows are summed in order with their rounding errors carried, so the
-    // result stays within a few units of the exact column sum even where the rows
-    // cancel (the ring's many short partial rows give the same by splitting).
-    float sw[VEC], sb[VEC], cw[VEC], cb[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) { sw[i] = 0.f; sb[i] = 0.f; cw[i] = 0.f; cb[i] = 0.f; }
-    auto kahan = [](float& s, float& c, float v) {
-      const float y = v - c;
-      const float t2 = s + y;
-      c = (t2 - s) - y;
-      s = t2;
-    };
-    if (live) {
-      // kSmallUnroll rows per batch, all their loads issued before the sums (rows
-      // past the end load row 0 and are skipped)
-      for (int64_t r0 = rl; r0 < rows; r0 += (int64_t)kSmallLanes * kSmallUnroll) {
-        float g[kSmallUnroll][VEC], xv[kSmallUnroll][VEC], rs[kSmallUnroll], mu[kSmallUnroll];
-#pragma unroll
-        for (int u = 0; u < kSmallUnroll; ++u) {
-          const int64_t r = r0 + (int64_t)u * kSmallLanes;
-          const int64_t rc = r < rows ? r : 0;
-          load_f32<T, VEC>(dy + rc * hidden + c0, g[u]);
-          load_f32<T, VEC>(x + rc * hidden + c0, xv[u]);
-          rs[u] = rstd[rc];
-          mu[u] = LN ? mean[rc] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < kSmallUnroll; ++u) {
-          if (r0 + (int64_t)u * kSmallLanes >= rows) break;
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            kahan(sw[i], cw[i], g[u][i] * ((xv[u][i] - mu[u]) * rs[u]));
-            if (LN) kahan(sb[i], cb[i], g[u][i]);
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      part[0][rl][p * VEC + i] = sw[i] - cw[i];
-      if (LN) part[1][rl][p * VEC + i] = sb[i] - cb[i];
-    }
-    __syncthreads();
-    if (t < kSmallPacks * VEC) {
-      const int col = (int)blockIdx.x * kSmallPacks * VEC + t;
-      float a[kSmallLanes], b[kSmallLanes];
-#pragma unroll
-      for (int l = 0; l < kSmallLanes; ++l) {
-        a[l] = part[0][l][t];
-        b[l] = LN ? part[1][l][t] : 0.f;
-      }
-#pragma unroll
-      for (int w2 = kSmallLanes / 2; w2 >= 1; w2 >>= 1)
-#pragma unroll
-        for (int l = 0; l < w2; ++l) {
-          a[l] += a[l + w2];
-          if (LN) b[l] += b[l + w2];
-        }
-      if (col < hidden) {
-        dweight[col] = from_f32<T>(a[0]);
-        if (LN) dbias[col] = from_f32<T>(b[0]);
-      }
-    }
-    return;
-  }
-  const int64_t r = (int64_t)blockIdx.x - ncolwg;
-  const T* dyr = dy + r * hidden;
-  const T* xr = x + r * hidden;
-  const float rs = rstd[r], mu = LN ? mean[r] : 0.f;
-  // pass 1: sum(g) (LayerNorm) and sum(g * xhat), g = dy * w
-  float sa = 0.f, sg = 0.f;
-  for (int c = t * VEC; c < hidden; c += kSmallBlock * VEC) {
-    float g[VEC], xv[VEC], wv[VEC];
-    load_f32<T, VEC>(dyr + c, g);
-    load_f32<T, VEC>(xr + c, xv);
-    load_f32<T, VEC>(w + c, wv);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      const float gi = g[i] * wv[i];
-      sa = __builtin_fmaf(gi, (xv[i] - mu) * rs, sa);
-      if (LN) sg += gi;
-    }
-  }
-  sa = wave_reduce(sa, SumOp());
-  if (LN) sg = wave_reduce(sg, SumOp());
-  if ((t & (kWave - 1)) == 0) {
-    red[0][t / kWave] = sa;
-    red[1][t / kWave] = sg;
-  }
-  __syncthreads();
-  float ta = red[0][0], tg = red[1][0];
-#pragma unroll
-  for (int k = 1; k < kSmallBlock / kWave; ++k) {
-    ta += red[0][k];
-    tg += red[1][k];
-  }
-  const float inv_h = 1.0f / (float)hidden;
-  const float mgx = ta * inv_h, mg = LN ? tg * inv_h : 0.f;
-  // pass 2: dx = rstd * (g - mean(g) - xhat * mean(g * xhat))   (RMSNorm: no mean(g))
-  for (int c = t * VEC; c < hidden; c += kSmallBlock * VEC) {
-    float g[VEC], xv[VEC], wv[VEC], o[VEC];
-    load_f32<T, VEC>(dyr + c, g);
-    load_f32<T, VEC>(xr + c, xv);
-    load_f32<T, VEC>(w + c, wv);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      const float xh = (xv[i] - mu) * rs;
-      o[i] = (g[i] * wv[i] - mg - xh * mgx) * rs;
-    }
-    store_f32<T, VEC>(dx + r * hidden + c, o);
-  }
 }
 
 template <bool LN>
@@ -1312,18 +1405,9 @@ static int norm_bwd_small_impl(const char* name, const void* dy, const void* x,
   }
   return EG_DISPATCH_FLOAT(dtype, name, [&] {
     using T = scalar_t;
-    constexpr int V = 16 / sizeof(T);
-    const int h = (int)hidden;
-    auto go = [&](auto vc) {
-      constexpr int VC = decltype(vc)::value;
-      const int ncol = (h + kSmallPacks * VC - 1) / (kSmallPacks * VC);
-      EG_LAUNCH((norm_bwd_small<T, VC, LN>), dim3((unsigned)(ncol + rows)), dim3(kSmallBlock), 0,
-                st, (const T*)dy, (const T*)x, (const T*)weight, mean, rstd, (T*)dx, (T*)dweight,
-                (T*)dbias, rows, h, ncol);
-      return check_launch(name);
-    };
-    if (vec_ok<T>(h, {dy, x, weight, dx})) return go(std::integral_constant<int, V>{});
-    return go(std::integral_constant<int, 1>{});
+    return launch_bwd_small<T, LN, false>((const T*)dy, (const T*)x, (const T*)nullptr,
+                                          (const T*)weight, mean, rstd, (T*)dx, (T*)dweight,
+                                          (T*)dbias, rows, (int)hidden, st, name);
   });
 }
 
