@@ -264,9 +264,10 @@ struct TileLoader {
   static constexpr int CPR = D / 8;
   static constexpr int ITER = ROWS * CPR / (64 * NW);
   static_assert(ITER >= 1 && ITER * 64 * NW == ROWS * CPR, "tile must split evenly over the waves");
-  int voff[ITER];
-  __device__ __forceinline__ void init() {
-    const int w = wave_id(), lane = threadIdx.x & 63;
+  int voff[ITER], w;  // w: this wave among the NW that load the tile
+  __device__ __forceinline__ void init(int wave) {
+    const int lane = threadIdx.x & 63;
+    w = wave;
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
       const int p = (it * NW + w) * 64 + lane;
@@ -280,7 +281,6 @@ struct TileLoader {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(slice + (int64_t)row0 * D), (short)0, (nrows - row0) * D * 2,
         0x00020000);
-    const int w = wave_id();
 #pragma unroll
     for (int it = 0; it < ITER; ++it)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (EG_LDS void*)(lds + (it * NW + w) * 64 * 8), 16,
@@ -316,8 +316,12 @@ __device__ __forceinline__ int query_head(int v, int BHkv, int group) {
 }
 
 // ------------------------------------------------------------------ forward
-template <typename T, int D, int NW, bool ROPE>
-__global__ __launch_bounds__(NW * 64, 2) void attn_fwd_kernel(
+// KG = 2: two groups of NW waves share the workgroup's rows and take the key tiles by
+// turns, each with tile buffers, a reference max, sums and an output of its own; group 1
+// hands these to group 0 through LDS at the end. Halves the chain of tiles of a row block,
+// which is what bounds a grid that leaves the chip's SIMDs with one wave or less.
+template <typename T, int D, int NW, int KG, bool ROPE>
+__global__ __launch_bounds__(NW * KG * 64, 2) void attn_fwd_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ o, float* __restrict__ lse, int S,
     float scale_log2, int nqb, int BH, int group, const float* __restrict__ rope_cos,
@@ -327,15 +331,16 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_kernel(
   constexpr int KSTEPS = D / 16, DT = D / 32;
   // One __shared__ object per buffer (see the file comment): LDS reads of one
   // buffer never wait for the loads in flight into the other.
-  __shared__ __align__(16) uint16_t Ks0[BN * D], Ks1[BN * D];
-  __shared__ __align__(16) uint16_t Vs0[BN * D], Vs1[BN * D];
+  __shared__ __align__(16) uint16_t Ks0[KG * BN * D], Ks1[KG * BN * D];
+  __shared__ __align__(16) uint16_t Vs0[KG * BN * D], Vs1[KG * BN * D];
 
   int vh, blk;
   block_coords(BH, vh, blk);
   if (vh >= BH) return;
   const int bh = query_head(vh, BH / group, group);
   const int q0 = (nqb - 1 - blk) * BM;  // longest rows first
-  const int lane = threadIdx.x & 63, w = wave_id();
+  const int lane = threadIdx.x & 63, w = wave_id() % NW, kg = wave_id() / NW;
+  const int kvo = kg * BN * D;  // this group's tile buffers
   const int l32 = lane & 31, hh = lane >> 5;
   const int64_t base = (int64_t)bh * S * D;
   const int64_t kvbase = (int64_t)(bh / group) * S * D;
@@ -373,17 +378,20 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_kernel(
   float m = -INFINITY, lsum = 0.f;
   const int kv_end = min(S, q0 + BM);
   const int ntiles = (kv_end + BN - 1) / BN;
+  const int nturns = (ntiles + KG - 1) / KG;  // tile KG * j + kg in turn j
   const int wave_first_row = q0 + 32 * w;
 
-  zero_lds<NW * 64>(Ks0, sizeof(Ks0));
-  zero_lds<NW * 64>(Ks1, sizeof(Ks1));
-  zero_lds<NW * 64>(Vs0, sizeof(Vs0));
-  zero_lds<NW * 64>(Vs1, sizeof(Vs1));
+  zero_lds<NW * KG * 64>(Ks0, sizeof(Ks0));
+  zero_lds<NW * KG * 64>(Ks1, sizeof(Ks1));
+  zero_lds<NW * KG * 64>(Vs0, sizeof(Vs0));
+  zero_lds<NW * KG * 64>(Vs1, sizeof(Vs1));
   __syncthreads();
   TileLoader<BN, D, NW> ld;
-  ld.init();
-  ld.load(kp, 0, S, Ks0);
-  ld.load(vp, 0, S, Vs0);
+  ld.init(w);
+  if (kg < ntiles) {
+    ld.load(kp, kg * BN, S, Ks0 + kvo);
+    ld.load(vp, kg * BN, S, Vs0 + kvo);
+  }
   // The rotation waits for q and the tables, so it comes after the first tile's
   // loads are issued: those are in flight meanwhile.
   if constexpr (ROPE)
@@ -392,14 +400,17 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_kernel(
     constexpr int buf = decltype(bufc)::value;
     wait_loads();
     __syncthreads();
-    if (j + 1 < ntiles) {
-      ld.load(kp, (j + 1) * BN, S, buf ? Ks0 : Ks1);
-      ld.load(vp, (j + 1) * BN, S, buf ? Vs0 : Vs1);
+    const int next = KG * (j + 1) + kg;
+    if (next < ntiles) {
+      ld.load(kp, next * BN, S, (buf ? Ks0 : Ks1) + kvo);
+      ld.load(vp, next * BN, S, (buf ? Vs0 : Vs1) + kvo);
     }
-    const int k0 = j * BN;
-    if (k0 > wave_first_row + 31) return;  // every key of the tile is above this wave's rows
-    const uint16_t* Kb = buf ? Ks1 : Ks0;
-    const uint16_t* Vb = buf ? Vs1 : Vs0;
+    const int k0 = (KG * j + kg) * BN;
+    // every key of the tile is above this wave's rows (a tile past the last one too)
+    if (k0 > wave_first_row + 31) return;
+    if (KG > 1 && k0 >= kv_end) return;
+    const uint16_t* Kb = (buf ? Ks1 : Ks0) + kvo;
+    const uint16_t* Vb = (buf ? Vs1 : Vs0) + kvo;
     f32x16 s[2];
     // S^T = K Q^T with the K operand reads kFwdPrefetch MFMAs ahead of their use
     // (MFMA i takes (kk, T2) = (i / 2, i % 2)); the scheduling groups keep that
@@ -495,9 +506,41 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_kernel(
       }
     }
   };
-  for (int j = 0; j < ntiles; j += 2) {
+  for (int j = 0; j < nturns; j += 2) {
     tile(std::integral_constant<int, 0>{}, j);
-    if (j + 1 < ntiles) tile(std::integral_constant<int, 1>{}, j + 1);
+    if (j + 1 < nturns) tile(std::integral_constant<int, 1>{}, j + 1);
+  }
+  if constexpr (KG > 1) {
+    // Group 1's values in the lane that holds the same rows in group 0, half of the output
+    // tiles in each K buffer.
+    constexpr int HT = DT / 2, STRIDE = NW * 64;
+    static_assert(HT * 16 * STRIDE * 4 <= (int)sizeof(Ks0), "half the output fits a buffer");
+    float* half0 = reinterpret_cast<float*>(Ks0);
+    float* half1 = reinterpret_cast<float*>(Ks1);
+    float* ml = reinterpret_cast<float*>(Vs0);
+    const int at = w * 64 + lane;
+    __syncthreads();  // the last tiles are consumed
+    if (kg == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          (t < HT ? half0 : half1)[((t % HT) * 16 + r) * STRIDE + at] = acc[t][r];
+      ml[at] = m;
+      ml[STRIDE + at] = lsum;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = ml[at], mx = fmaxf(m, m1), ref = mx == -INFINITY ? 0.f : mx;
+    const float a0 = __builtin_amdgcn_exp2f(m - ref), a1 = __builtin_amdgcn_exp2f(m1 - ref);
+    lsum = lsum * a0 + ml[STRIDE + at] * a1;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[t][r] = acc[t][r] * a0 +
+                    (t < HT ? half0 : half1)[((t % HT) * 16 + r) * STRIDE + at] * a1;
+    m = mx;
   }
 
   const float ltot = lsum + __shfl_xor(lsum, 32, 64);
@@ -584,7 +627,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dkdv_kernel(
   const int s_begin = min(nsteps, pi * per), s_end = min(nsteps, s_begin + per);
   const int wave_first_key = k0 + 32 * w;
   TileLoader<BQ, D, NW> ld;
-  ld.init();
+  ld.init(w);
   auto qhead = [&](int step) { return kvh * group + step / ntq; };
   auto qtile = [&](int step) { return i_first + step % ntq; };
   // lse and delta of a tile's rows: wave 0 loads them when the tile is requested
@@ -611,7 +654,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dkdv_kernel(
   __syncthreads();
   {
     TileLoader<BK, D, NW> lv;  // keys past S stay zero
-    lv.init();
+    lv.init(w);
     lv.load(v + base, k0, S, Vk);
   }
   if (s_begin < s_end) {
@@ -800,8 +843,9 @@ __global__ __launch_bounds__(256) void attn_dkdv_reduce_kernel(const float* __re
 }
 
 // ------------------------------------------------------------------- dQ
-template <typename T, int D, int NW, bool ROPE>
-__global__ __launch_bounds__(NW * 64, 2) void attn_dq_kernel(
+// KG as in the forward.
+template <typename T, int D, int NW, int KG, bool ROPE>
+__global__ __launch_bounds__(NW * KG * 64, 2) void attn_dq_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const uint16_t* __restrict__ dout,
     const uint16_t* __restrict__ o, const float* __restrict__ lse, float* __restrict__ delta,
@@ -810,15 +854,17 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dq_kernel(
   using v8 = typename MM<T>::v8;
   constexpr int BM = 32 * NW, BN = 64;
   constexpr int KSTEPS = D / 16, DT = D / 32;
-  __shared__ __align__(16) uint16_t Ks0[BN * D], Ks1[BN * D];  // one object per buffer
-  __shared__ __align__(16) uint16_t Vs0[BN * D], Vs1[BN * D];
+  // one object per buffer
+  __shared__ __align__(16) uint16_t Ks0[KG * BN * D], Ks1[KG * BN * D];
+  __shared__ __align__(16) uint16_t Vs0[KG * BN * D], Vs1[KG * BN * D];
 
   int vh, blk;
   block_coords(BH, vh, blk);
   if (vh >= BH) return;
   const int bh = query_head(vh, BH / group, group);
   const int q0 = (nqb - 1 - blk) * BM;
-  const int lane = threadIdx.x & 63, w = wave_id();
+  const int lane = threadIdx.x & 63, w = wave_id() % NW, kg = wave_id() / NW;
+  const int kvo = kg * BN * D;  // this group's tile buffers
   const int l32 = lane & 31, hh = lane >> 5;
   const int64_t base = (int64_t)bh * S * D;
   const int64_t kvbase = (int64_t)(bh / group) * S * D;
@@ -849,13 +895,14 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dq_kernel(
   const float lv = lse[(int64_t)bh * S + qrc];
   const float l2 = qrow < S ? lv * kLog2e : INFINITY;
   const float dl = qrow < S ? dsum : 0.f;
-  if (qrow < S && hh == 0) delta[(int64_t)bh * S + qrow] = dsum;
+  if (qrow < S && hh == 0 && kg == 0) delta[(int64_t)bh * S + qrow] = dsum;
 
   f32x16 acc[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) acc[t] = f32x16{};
   const int kv_end = min(S, q0 + BM);
   const int ntiles = (kv_end + BN - 1) / BN;
+  const int nturns = (ntiles + KG - 1) / KG;
   const int wave_first_row = q0 + 32 * w;
   const uint16_t* kp = k + kvbase;
   const uint16_t* vp = v + kvbase;
@@ -875,27 +922,31 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dq_kernel(
       offV[t][1] = toff<D>(r0 + 8, col >> 3) + (col & 7);
     }
   }
-  zero_lds<NW * 64>(Ks0, sizeof(Ks0));
-  zero_lds<NW * 64>(Ks1, sizeof(Ks1));
-  zero_lds<NW * 64>(Vs0, sizeof(Vs0));
-  zero_lds<NW * 64>(Vs1, sizeof(Vs1));
+  zero_lds<NW * KG * 64>(Ks0, sizeof(Ks0));
+  zero_lds<NW * KG * 64>(Ks1, sizeof(Ks1));
+  zero_lds<NW * KG * 64>(Vs0, sizeof(Vs0));
+  zero_lds<NW * KG * 64>(Vs1, sizeof(Vs1));
   __syncthreads();
   TileLoader<BN, D, NW> ld;
-  ld.init();
-  ld.load(kp, 0, S, Ks0);
-  ld.load(vp, 0, S, Vs0);
+  ld.init(w);
+  if (kg < ntiles) {
+    ld.load(kp, kg * BN, S, Ks0 + kvo);
+    ld.load(vp, kg * BN, S, Vs0 + kvo);
+  }
   auto tile = [&](auto bufc, int j) {
     constexpr int buf = decltype(bufc)::value;
     wait_loads();
     __syncthreads();
-    if (j + 1 < ntiles) {
-      ld.load(kp, (j + 1) * BN, S, buf ? Ks0 : Ks1);
-      ld.load(vp, (j + 1) * BN, S, buf ? Vs0 : Vs1);
+    const int next = KG * (j + 1) + kg;
+    if (next < ntiles) {
+      ld.load(kp, next * BN, S, (buf ? Ks0 : Ks1) + kvo);
+      ld.load(vp, next * BN, S, (buf ? Vs0 : Vs1) + kvo);
     }
-    const int k0 = j * BN;
+    const int k0 = (KG * j + kg) * BN;
     if (k0 > wave_first_row + 31) return;
-    const uint16_t* Kb = buf ? Ks1 : Ks0;
-    const uint16_t* Vb = buf ? Vs1 : Vs0;
+    if (KG > 1 && k0 >= kv_end) return;
+    const uint16_t* Kb = (buf ? Ks1 : Ks0) + kvo;
+    const uint16_t* Vb = (buf ? Vs1 : Vs0) + kvo;
     f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
     // S^T = K Q^T and dP^T = V dO^T interleaved, each operand read kDqPrefetch MFMAs
     // ahead (read i: kk = i / 4, T2 = (i / 2) % 2, K for even i and V for odd i);
@@ -961,9 +1012,31 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_dq_kernel(
       }
     }
   };
-  for (int j = 0; j < ntiles; j += 2) {
+  for (int j = 0; j < nturns; j += 2) {
     tile(std::integral_constant<int, 0>{}, j);
-    if (j + 1 < ntiles) tile(std::integral_constant<int, 1>{}, j + 1);
+    if (j + 1 < nturns) tile(std::integral_constant<int, 1>{}, j + 1);
+  }
+  if constexpr (KG > 1) {
+    constexpr int HT = DT / 2, STRIDE = NW * 64;
+    static_assert(HT * 16 * STRIDE * 4 <= (int)sizeof(Ks0), "half of dQ fits a buffer");
+    float* half0 = reinterpret_cast<float*>(Ks0);
+    float* half1 = reinterpret_cast<float*>(Ks1);
+    const int at = w * 64 + lane;
+    __syncthreads();  // the last tiles are consumed
+    if (kg == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          (t < HT ? half0 : half1)[((t % HT) * 16 + r) * STRIDE + at] = acc[t][r];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[t][r] += (t < HT ? half0 : half1)[((t % HT) * 16 + r) * STRIDE + at];
   }
 
   if (qrow < S) {
@@ -1011,6 +1084,25 @@ int dkdv_parts(int64_t BHkv, int64_t S, int64_t D) {
   if (wgs <= 0 || wgs >= kDkdvTarget) return 1;
   return (int)std::min<int64_t>(kDkdvMaxParts, (kDkdvTarget + wgs - 1) / wgs);
 }
+// Parts to take, up to that bound (which sizes the workspace): each costs the write and
+// read of its slabs, and shortens the longest walk until the chip is full (two workgroups
+// per CU). About 1.1 us per 32-row step and 5 TB/s fit the measured backward calls: bf16
+// [2, 12, 1000, 64] 55.0 us in 6 parts, 46.8 in 3, 48.6 in 2; [4, 8, 512, 128] 72.0 in 8, 51.2
+// in 4, 46.6 in 2; [1, 32 / 8, 2048, 128] 180.7 in 8, 168.8 in 6, 173.5 in 4; [1, 4, 8192, 64]
+// 225.5 in 4, 261.2 in 2.
+int dkdv_split(int64_t BHkv, int64_t group, int64_t S, int64_t D) {
+  const int most = dkdv_parts(BHkv, S, D);
+  const double steps = (double)group * (double)((S + 31) / 32);  // the longest walk
+  const double wgs = (double)BHkv * (double)((S + 127) / 128);
+  const double full = wgs * steps / 2 / 512, slab = 16e-6 / 5 * (double)BHkv * (double)(S * D);
+  int best = 1;
+  double least = 0;
+  for (int p = 1; p <= most; ++p) {
+    const double c = 1.1 * std::max(steps / p, full) + (p > 1 ? slab * p : 0.0);
+    if (p == 1 || c < least) least = c, best = p;
+  }
+  return best;
+}
 // Backward workspace after delta (fp32 [BH, S], rounded up to 256 bytes): the split
 // walk's slabs, 2 x parts x BHkv x S x D fp32 (none without a split).
 size_t attn_delta_bytes(int64_t BH, int64_t S) { return ((size_t)(BH * S) * 4 + 255) / 256 * 256; }
@@ -1053,24 +1145,38 @@ inline unsigned grid_for(int64_t BH, int nblocks) {
   return (unsigned)(((BH + 7) / 8) * 8 * nblocks);
 }
 
+// Two key groups per workgroup (KG = 2) in the forward and dQ: for grids of at most 512
+// 128-row workgroups, where the chain of key tiles of the last rows sets the time, from
+// 768 positions (12 tiles) on. bf16 forward / backward, one group against two: [1, 16 / 4,
+// 2000, 128] 38.2 / 116.9 -> 31.8 / 108.1 us, [1, 4 / 2, 4096, 128] 69.7 / 167.4 -> 54.9 /
+// 145.1, [1, 4, 8192, 64] 107.3 / 225.8 -> 89.0 / 207.2; shorter rows only pay for the
+// exchange ([1, 2 / 1, 200, 128] 8.2 -> 9.0 us, [4, 8, 512, 128] 12.8 -> 13.3).
+constexpr int64_t kSplitKeysGrid = 512, kSplitKeysSeq = 768;
+inline bool split_keys(int64_t BH, int64_t S) {
+  return S >= kSplitKeysSeq && grid_for(BH, (int)((S + 127) / 128)) <= kSplitKeysGrid;
+}
+
 // With ROPE, q is rotated in registers by the fp32 tables rc/rs [S, D] as it is
 // loaded (k must already be rotated).
 template <typename T, int D, bool ROPE = false>
 int attn_fwd_launch(const void* q, const void* k, const void* v, void* o, float* lse, int64_t BH,
                     int64_t S, int group, float scale, hipStream_t st,
                     const float* rc = nullptr, const float* rs = nullptr) {
-  auto go = [&](auto nwc) {
-    constexpr int NW = decltype(nwc)::value;
+  auto go = [&](auto nwc, auto kgc) {
+    constexpr int NW = decltype(nwc)::value, KG = decltype(kgc)::value;
     const int nqb = (int)((S + 32 * NW - 1) / (32 * NW));
-    EG_LAUNCH((attn_fwd_kernel<T, D, NW, ROPE>), dim3(grid_for(BH, nqb)), dim3(NW * 64), 0, st,
+    EG_LAUNCH((attn_fwd_kernel<T, D, NW, KG, ROPE>), dim3(grid_for(BH, nqb)), dim3(NW * KG * 64), 0, st,
               (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse,
               (int)S, scale * kLog2e, nqb, (int)BH, group, rc, rs);
     return check_launch("eg_attn_fwd");
   };
   const int nqb_full = (int)((S + 32 * kFwdWaves - 1) / (32 * kFwdWaves));
+  using One = std::integral_constant<int, 1>;
+  if (split_keys(BH, S))
+    return go(std::integral_constant<int, kFwdSmallWaves>{}, std::integral_constant<int, 2>{});
   if (grid_for(BH, nqb_full) < (unsigned)kFwdFullGrid)
-    return go(std::integral_constant<int, kFwdSmallWaves>{});
-  return go(std::integral_constant<int, kFwdWaves>{});
+    return go(std::integral_constant<int, kFwdSmallWaves>{}, One{});
+  return go(std::integral_constant<int, kFwdWaves>{}, One{});
 }
 
 // BH counts query heads (x batch); the key/value tensors hold BH / group heads.
@@ -1087,16 +1193,21 @@ int attn_bwd_launch(const void* dout, const void* q, const void* k, const void* 
   // dK/dV kernel reads.
   constexpr int NQ = kDqWaves;
   const int nqb = (int)((S + 32 * NQ - 1) / (32 * NQ));
-  EG_LAUNCH((attn_dq_kernel<T, D, NQ, ROPE>), dim3(grid_for(BH, nqb)), dim3(NQ * 64), 0, st,
-            (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout,
-            (const uint16_t*)o, lse, delta, (uint16_t*)dq, (int)S, scale, scale * kLog2e, nqb,
-            (int)BH, group, rc, rs);
+  auto run_dq = [&](auto kgc) {
+    constexpr int KG = decltype(kgc)::value;
+    EG_LAUNCH((attn_dq_kernel<T, D, NQ, KG, ROPE>), dim3(grid_for(BH, nqb)), dim3(NQ * KG * 64), 0,
+              st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
+              (const uint16_t*)dout, (const uint16_t*)o, lse, delta, (uint16_t*)dq, (int)S, scale,
+              scale * kLog2e, nqb, (int)BH, group, rc, rs);
+  };
+  if (split_keys(BH, S)) run_dq(std::integral_constant<int, 2>{});
+  else run_dq(std::integral_constant<int, 1>{});
   if (int rc = check_launch("eg_attn_bwd(dq)")) return rc;
   constexpr int NK = dkdv_waves<D>();
   const int nkb = (int)((S + 32 * NK - 1) / (32 * NK));
   const int64_t BHkv = BH / group;
   static_assert(NK == dkdv_waves<128>(), "dkdv_parts assumes one key-block width");
-  const int parts = dkdv_parts(BHkv, S, D);
+  const int parts = dkdv_split(BHkv, group, S, D);
   EG_LAUNCH((attn_dkdv_kernel<T, D, NK, kDkdvRows, ROPE>), dim3(grid_for(BHkv * parts, nkb)),
             dim3(NK * 64), 0, st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
             (const uint16_t*)dout, lse, delta, (uint16_t*)dk, (uint16_t*)dv, (int)S, scale,
@@ -1113,17 +1224,24 @@ int attn_bwd_launch(const void* dout, const void* q, const void* k, const void* 
 // templates without a host launch stub (undefined symbol at load time); naming
 // every kernel here makes the stubs certain.
 #define EG_ATTN_INSTANTIATE(T, D, R)                                                         \
-  template __global__ void attn_fwd_kernel<T, D, kFwdWaves, R>(                              \
+  template __global__ void attn_fwd_kernel<T, D, kFwdWaves, 1, R>(                           \
       const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, float*, int, float, int,   \
       int, int, const float*, const float*);                                                 \
-  template __global__ void attn_fwd_kernel<T, D, kFwdSmallWaves, R>(                         \
+  template __global__ void attn_fwd_kernel<T, D, kFwdSmallWaves, 1, R>(                      \
+      const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, float*, int, float, int,   \
+      int, int, const float*, const float*);                                                 \
+  template __global__ void attn_fwd_kernel<T, D, kFwdSmallWaves, 2, R>(                      \
       const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, float*, int, float, int,   \
       int, int, const float*, const float*);                                                 \
   template __global__ void attn_dkdv_kernel<T, D, dkdv_waves<D>(), kDkdvRows, R>(            \
       const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const float*,        \
       const float*, uint16_t*, uint16_t*, int, float, float, int, int, const float*,           \
       const float*, int, float*);                                                            \
-  template __global__ void attn_dq_kernel<T, D, kDqWaves, R>(                                \
+  template __global__ void attn_dq_kernel<T, D, kDqWaves, 1, R>(                                \
+      const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*,     \
+      const float*, float*, uint16_t*, int, float, float, int, int, int, const float*,         \
+      const float*);                                                                      \
+  template __global__ void attn_dq_kernel<T, D, kDqWaves, 2, R>(                                \
       const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*,     \
       const float*, float*, uint16_t*, int, float, float, int, int, int, const float*,         \
       const float*);
