@@ -27,8 +27,8 @@
 // over the other side is cut over the kGenWaves waves of a workgroup (tile t to wave
 // t % kGenWaves), which add their parts through LDS in wave order; the dK/dV walk is
 // also cut over `parts` workgroups whose fp32 slabs attn_gen_reduce_kernel adds in
-// order. At fp32 [1, 8 / 2 kv, 1024, 64] the kernels take 25 us (forward), 40 us (dQ)
-// and 51 + 5 us (dK/dV and its reduction), against 6031, 6316 and 30931 us for one wave per
+// order. At fp32 [1, 8 / 2 kv, 1024, 64] the kernels take 22 us (forward), 33 us (dQ)
+// and 43 + 5 us (dK/dV and its reduction), against 6031, 6316 and 30931 us for one wave per
 // 64 rows on VALU FMAs (128 waves on the chip's 1024 SIMDs, about 6 us per key of the
 // longest row: one dependent chain with its operands broadcast from LDS).
 // No atomics: every sum has a fixed order.
@@ -49,6 +49,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kGenWaves = 4;
 constexpr int kGenThreads = kGenWaves * 64;
+constexpr int64_t kGenTarget = 512;  // workgroups: two per CU
 constexpr float kGenLog2e = 1.4426950408889634f;
 constexpr float kGenLn2 = 0.6931471805599453f;
 
@@ -185,6 +186,17 @@ inline dim3 gen_grid(int64_t x, int64_t blocks) {
   return dim3((unsigned)x, (unsigned)y, (unsigned)((blocks + y - 1) / y));
 }
 
+// Order in which the blocks of a triangle are taken, 0 = the longest walk. Longest first,
+// so that what a CU takes last is short. Where the whole grid is resident at once, two
+// workgroups on a CU (kGenTarget), nothing is taken last: the second of each pair then
+// comes shortest first, so that every CU holds a long and a short walk
+// (fp32 [1, 8 / 2 kv, 1024, 64], 512 workgroups: 25, 40 and 51 us longest first throughout,
+// 22, 33 and 43 us so; the longest CU had 1.5 times the mean work).
+__device__ __forceinline__ int walk_order(int blk, int n) {
+  const int first = kGenTarget / 2 / gridDim.x;  // blocks of the first workgroup on each CU
+  return (int64_t)gridDim.x * n <= kGenTarget && blk >= first ? n - 1 - (blk - first) : blk;
+}
+
 __device__ __forceinline__ float over_groups(float v, bool is_max) {
 #pragma unroll
   for (int off = 16; off <= 32; off <<= 1) {
@@ -205,7 +217,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attn_gen_fwd_kernel(
   __shared__ float wm[kGenWaves][16], wl[kGenWaves][16];
   const int bh = blockIdx.x, blk = block_index();
   if (blk >= nqb) return;
-  const int q0 = (nqb - 1 - blk) * 16;
+  const int q0 = (nqb - 1 - walk_order(blk, nqb)) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const T* qs = q + (int64_t)bh * S * D;
   const T* ks = k + (int64_t)(bh / group) * S * D;
@@ -305,7 +317,7 @@ __global__ __launch_bounds__(kGenThreads, DM > 64 ? 1 : 2) void attn_gen_dq_kern
   __shared__ float buf[kGenWaves][16][DM + 4];
   const int bh = blockIdx.x, blk = block_index();
   if (blk >= nqb) return;
-  const int q0 = (nqb - 1 - blk) * 16;
+  const int q0 = (nqb - 1 - walk_order(blk, nqb)) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const int query = q0 + m16, qc = min(query, S - 1);
   const int64_t row = ((int64_t)bh * S + qc) * D;
@@ -389,8 +401,9 @@ __global__ __launch_bounds__(kGenThreads, DM > 64 ? 1 : 2) void attn_gen_dkdv_ke
   constexpr int NS = DM / 4, DT = DM / 16;
   __shared__ float buf[kGenWaves][16][DM + 4];
   const int bhk = blockIdx.x % BHkv, pi = blockIdx.x / BHkv;
-  const int k0 = block_index() * 16;  // the longest walks first
-  if (k0 >= S) return;
+  const int nkb = (S + 15) / 16, blk = block_index();
+  if (blk >= nkb) return;
+  const int k0 = walk_order(blk, nkb) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const int key = k0 + m16;
   const int64_t slice = (int64_t)S * D;
@@ -503,7 +516,7 @@ int gen_dispatch(int dtype, int64_t D, std::initializer_list<const void*> ptrs, 
 
 // Parts of the dK/dV walk: at least kGenTarget workgroups (two per CU), while the
 // longest walk still gives every wave kGenMinSteps steps. From the shape only.
-constexpr int64_t kGenTarget = 512, kGenMaxParts = 8, kGenMinSteps = 2;
+constexpr int64_t kGenMaxParts = 8, kGenMinSteps = 2;
 int64_t gen_parts(int64_t BHkv, int64_t group, int64_t S) {
   const int64_t nkb = (S + 15) / 16;
   const int64_t want = (kGenTarget + BHkv * nkb - 1) / (BHkv * nkb);

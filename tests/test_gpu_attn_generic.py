@@ -30,9 +30,11 @@ def test_generic_attention_edges(B, H, KVH, S, D, dtype):
     assert rep.ok, "\n".join(rep.failures())
 
 
+# 40 heads of 130 rows: a grid resident at once, whose second half runs shortest first.
+@pytest.mark.parametrize("H,KVH,S", ((4, 2, 200), (40, 10, 130)))
 @pytest.mark.parametrize("D", (64, 128))
-def test_generic_attention_fp32_wide_heads(D):
-    w = Workload(dims=dict(B=1, H=4, KVH=2, S=200, D=D), dtype="float32")
+def test_generic_attention_fp32_wide_heads(D, H, KVH, S):
+    w = Workload(dims=dict(B=1, H=H, KVH=KVH, S=S, D=D), dtype="float32")
     print("\n[gpu-attn-generic]", w.dims, flush=True)
     rep = verify(OP, pair_module("causal_attention_gqa"), device="cuda", workloads=(w,))
     assert rep.ok, "\n".join(rep.failures())
