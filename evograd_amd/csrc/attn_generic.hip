@@ -187,14 +187,18 @@ inline dim3 gen_grid(int64_t x, int64_t blocks) {
 }
 
 // Order in which the blocks of a triangle are taken, 0 = the longest walk. Longest first,
-// so that what a CU takes last is short. Where the whole grid is resident at once, two
-// workgroups on a CU (kGenTarget), nothing is taken last: the second of each pair then
-// comes shortest first, so that every CU holds a long and a short walk
-// (fp32 [1, 8 / 2 kv, 1024, 64], 512 workgroups: 25, 40 and 51 us longest first throughout,
-// 22, 33 and 43 us so; the longest CU had 1.5 times the mean work).
+// so that what a CU takes last is short. PAIR, for kernels with two workgroups on a CU:
+// where the whole grid is resident at once (kGenTarget), nothing is taken last and the
+// second workgroup of each CU comes shortest first, so that every CU holds a long and a
+// short walk. fp32, longest first against paired: [1, 8 / 2 kv, 1024, 64] forward 23.6 ->
+// 19.7 us, backward 87.4 -> 73.0 (the longest CU had 1.5 times the mean work), [1, 8 / 2,
+// 1000, 128] forward 44.8 -> 37.2; the backward there has registers for one workgroup on
+// a CU and would go 176.6 -> 189.9.
+template <bool PAIR>
 __device__ __forceinline__ int walk_order(int blk, int n) {
   const int first = kGenTarget / 2 / gridDim.x;  // blocks of the first workgroup on each CU
-  return (int64_t)gridDim.x * n <= kGenTarget && blk >= first ? n - 1 - (blk - first) : blk;
+  return PAIR && (int64_t)gridDim.x * n <= kGenTarget && blk >= first ? n - 1 - (blk - first)
+                                                                      : blk;
 }
 
 __device__ __forceinline__ float over_groups(float v, bool is_max) {
@@ -217,7 +221,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void attn_gen_fwd_kernel(
   __shared__ float wm[kGenWaves][16], wl[kGenWaves][16];
   const int bh = blockIdx.x, blk = block_index();
   if (blk >= nqb) return;
-  const int q0 = (nqb - 1 - walk_order(blk, nqb)) * 16;
+  const int q0 = (nqb - 1 - walk_order<true>(blk, nqb)) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const T* qs = q + (int64_t)bh * S * D;
   const T* ks = k + (int64_t)(bh / group) * S * D;
@@ -317,7 +321,7 @@ __global__ __launch_bounds__(kGenThreads, DM > 64 ? 1 : 2) void attn_gen_dq_kern
   __shared__ float buf[kGenWaves][16][DM + 4];
   const int bh = blockIdx.x, blk = block_index();
   if (blk >= nqb) return;
-  const int q0 = (nqb - 1 - walk_order(blk, nqb)) * 16;
+  const int q0 = (nqb - 1 - walk_order<(DM <= 64)>(blk, nqb)) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const int query = q0 + m16, qc = min(query, S - 1);
   const int64_t row = ((int64_t)bh * S + qc) * D;
@@ -403,7 +407,7 @@ __global__ __launch_bounds__(kGenThreads, DM > 64 ? 1 : 2) void attn_gen_dkdv_ke
   const int bhk = blockIdx.x % BHkv, pi = blockIdx.x / BHkv;
   const int nkb = (S + 15) / 16, blk = block_index();
   if (blk >= nkb) return;
-  const int k0 = walk_order(blk, nkb) * 16;
+  const int k0 = walk_order<(DM <= 64)>(blk, nkb) * 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m16 = lane & 15, g = lane >> 4;
   const int key = k0 + m16;
   const int64_t slice = (int64_t)S * D;
