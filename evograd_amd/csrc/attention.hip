@@ -34,13 +34,15 @@
 //
 // Kernels (all deterministic, no atomics):
 //   attn_fwd:   workgroup = 8 waves x 32 query rows (4 waves on grids of fewer than
-//               512 8-wave workgroups); double-buffered 64-key K and
+//               512 8-wave workgroups; 2 x 4 waves cutting the keys between them on
+//               small grids of long rows, split_keys); double-buffered 64-key K and
 //               V tiles; online softmax in the log2 domain against a running
 //               reference max, refreshed only when a P term could exceed 2^8 (a
 //               lane's sum of P terms bounds each term, so no per-tile max is
 //               formed; exact: the reference point cancels in o = sum / l);
 //               S^T = K Q^T, O^T += V^T P^T.
-//   attn_dq:    (runs first) workgroup = 4 waves x 32 query rows; also computes
+//   attn_dq:    (runs first) workgroup = 4 waves x 32 query rows (or 2 x 4 waves, as
+//               above); also computes
 //               delta = rowsum(do * o) for its rows into the workspace;
 //               double-buffered 64-key K, V tiles; S^T = K Q^T, dP^T = V dO^T,
 //               dQ^T += K^T dS^T.
