@@ -341,7 +341,8 @@ __global__ __launch_bounds__(NW * KG * 64, 2) void attn_fwd_kernel(
   if (vh >= BH) return;
   const int bh = query_head(vh, BH / group, group);
   const int q0 = (nqb - 1 - blk) * BM;  // longest rows first
-  const int lane = threadIdx.x & 63, w = wave_id() % NW, kg = wave_id() / NW;
+  const int lane = threadIdx.x & 63;
+  const int w = KG == 1 ? wave_id() : wave_id() % NW, kg = KG == 1 ? 0 : wave_id() / NW;
   const int kvo = kg * BN * D;  // this group's tile buffers
   const int l32 = lane & 31, hh = lane >> 5;
   const int64_t base = (int64_t)bh * S * D;
@@ -865,7 +866,8 @@ __global__ __launch_bounds__(NW * KG * 64, 2) void attn_dq_kernel(
   if (vh >= BH) return;
   const int bh = query_head(vh, BH / group, group);
   const int q0 = (nqb - 1 - blk) * BM;
-  const int lane = threadIdx.x & 63, w = wave_id() % NW, kg = wave_id() / NW;
+  const int lane = threadIdx.x & 63;
+  const int w = KG == 1 ? wave_id() : wave_id() % NW, kg = KG == 1 ? 0 : wave_id() / NW;
   const int kvo = kg * BN * D;  // this group's tile buffers
   const int l32 = lane & 31, hh = lane >> 5;
   const int64_t base = (int64_t)bh * S * D;
@@ -1086,21 +1088,23 @@ int dkdv_parts(int64_t BHkv, int64_t S, int64_t D) {
   if (wgs <= 0 || wgs >= kDkdvTarget) return 1;
   return (int)std::min<int64_t>(kDkdvMaxParts, (kDkdvTarget + wgs - 1) / wgs);
 }
-// Parts to take, up to that bound (which sizes the workspace): each costs the write and
-// read of its slabs, and shortens the longest walk until the chip is full (two workgroups
-// per CU). About 1.1 us per 32-row step and 5 TB/s fit the measured backward calls: bf16
-// [2, 12, 1000, 64] 55.0 us in 6 parts, 46.8 in 3, 48.6 in 2; [4, 8, 512, 128] 72.0 in 8, 51.2
-// in 4, 46.6 in 2; [1, 32 / 8, 2048, 128] 180.7 in 8, 168.8 in 6, 173.5 in 4; [1, 4, 8192, 64]
-// 225.5 in 4, 261.2 in 2.
+// Parts to take, up to that bound (which sizes the workspace): each shortens the longest
+// walk until the chip is full (two workgroups per CU) and costs its slabs' write and read.
+// In us, 1.1 (D = 128) or 0.9 (64) per 32-row step, 1.6 per million elements of dK and
+// part, and 5 for the reduction: fitted over 48 shapes timed at every number of parts; the
+// backward at the choice against at the bound: bf16 [2, 12, 1000, 64] 52.4 -> 44.6 us in 3
+// parts, [4, 8, 512, 128] 72.9 -> 45.8 in 1, [1, 8, 2048, 128] 106.6 -> 91.2 in 3 (88.0 in 4),
+// [1, 32 / 8, 512, 128] 46.8 in 8 (49.2 in 6), [1, 4, 8192, 64] 207.6 in 4 (241.9 in 2).
 int dkdv_split(int64_t BHkv, int64_t group, int64_t S, int64_t D) {
   const int most = dkdv_parts(BHkv, S, D);
+  const double step = D == 128 ? 1.1 : 0.9;
   const double steps = (double)group * (double)((S + 31) / 32);  // the longest walk
   const double wgs = (double)BHkv * (double)((S + 127) / 128);
-  const double full = wgs * steps / 2 / 512, slab = 16e-6 / 5 * (double)BHkv * (double)(S * D);
+  const double full = wgs * steps / 2 / 512, slab = 1.6e-6 * (double)BHkv * (double)(S * D);
   int best = 1;
   double least = 0;
   for (int p = 1; p <= most; ++p) {
-    const double c = 1.1 * std::max(steps / p, full) + (p > 1 ? slab * p : 0.0);
+    const double c = step * std::max(steps / p, full) + (p > 1 ? slab * p + 5.0 : 0.0);
     if (p == 1 || c < least) least = c, best = p;
   }
   return best;
