@@ -1157,9 +1157,18 @@ inline unsigned grid_for(int64_t BH, int nblocks) {
 // 2000, 128] 38.2 / 116.9 -> 31.8 / 108.1 us, [1, 4 / 2, 4096, 128] 69.7 / 167.4 -> 54.9 /
 // 145.1, [1, 4, 8192, 64] 107.3 / 225.8 -> 89.0 / 207.2; shorter rows only pay for the
 // exchange ([1, 2 / 1, 200, 128] 8.2 -> 9.0 us, [4, 8, 512, 128] 12.8 -> 13.3).
+// A CU holds one workgroup of two groups or two of one, so past 256 workgroups the second
+// round has to be won back by longer rows: forward at D = 128 [1, 64 / 8, 1000] 28.0 -> 30.1
+// us but [1, 32 / 8, 2048] 46.7 -> 43.9, at 64 always ahead ([1, 40 / 8, 1000] 16.9 -> 15.5);
+// backward at 128 [1, 48 / 12, 903] 90.5 -> 97.0, [1, 32 / 8, 2048] 178.1 -> 180.9, but
+// [1, 24 / 8, 2048] 154.6 -> 151.3 and [1, 16 / 4, 4096] 290.4 -> 281.7, at 64 [1, 32 / 8,
+// 1800] (480 workgroups) 84.5 -> 85.2 but [2, 24 / 8, 1024] (384) 61.1 -> 59.5.
 constexpr int64_t kSplitKeysGrid = 512, kSplitKeysSeq = 768;
-inline bool split_keys(int64_t BH, int64_t S) {
-  return S >= kSplitKeysSeq && grid_for(BH, (int)((S + 127) / 128)) <= kSplitKeysGrid;
+inline bool split_keys(int64_t BH, int64_t S, int64_t D, bool dq) {
+  const int64_t grid = grid_for(BH, (int)((S + 127) / 128));
+  if (S < kSplitKeysSeq || grid > kSplitKeysGrid) return false;
+  const bool longer = D == 64 || S >= 2048;
+  return grid <= 256 || (dq ? S >= 4096 || (grid <= 384 && longer) : longer);
 }
 
 // With ROPE, q is rotated in registers by the fp32 tables rc/rs [S, D] as it is
@@ -1178,7 +1187,7 @@ int attn_fwd_launch(const void* q, const void* k, const void* v, void* o, float*
   };
   const int nqb_full = (int)((S + 32 * kFwdWaves - 1) / (32 * kFwdWaves));
   using One = std::integral_constant<int, 1>;
-  if (split_keys(BH, S))
+  if (split_keys(BH, S, D, false))
     return go(std::integral_constant<int, kFwdSmallWaves>{}, std::integral_constant<int, 2>{});
   if (grid_for(BH, nqb_full) < (unsigned)kFwdFullGrid)
     return go(std::integral_constant<int, kFwdSmallWaves>{}, One{});
@@ -1206,7 +1215,7 @@ int attn_bwd_launch(const void* dout, const void* q, const void* k, const void* 
               (const uint16_t*)dout, (const uint16_t*)o, lse, delta, (uint16_t*)dq, (int)S, scale,
               scale * kLog2e, nqb, (int)BH, group, rc, rs);
   };
-  if (split_keys(BH, S)) run_dq(std::integral_constant<int, 2>{});
+  if (split_keys(BH, S, D, true)) run_dq(std::integral_constant<int, 2>{});
   else run_dq(std::integral_constant<int, 1>{});
   if (int rc = check_launch("eg_attn_bwd(dq)")) return rc;
   constexpr int NK = dkdv_waves<D>();
