@@ -981,7 +981,8 @@ __global__ __launch_bounds__(kSmallBlock) void norm_bwd_small(
     auto kahan = [](float& s, float& c, float v) {
       const float y = v - c;
       const float t2 = s + y;
-      c = (t2 - s) - y;
+      // an infinite or NaN sum goes on as a plain one: inf - inf is no correction
+      c = __builtin_fabsf(t2) < INFINITY ? (t2 - s) - y : 0.f;
       s = t2;
     };
     if (live) {

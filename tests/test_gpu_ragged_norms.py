@@ -59,3 +59,48 @@ def test_norms_ragged_rows(op, rows, cols, offset, dtype):
     _close(grads[n], (gd * xhat).sum(0), dtype, (gd * xhat).abs().sum(0) + 1)
     if op == "layernorm":
         _close(grads[2], gd.sum(0), dtype, gd.abs().sum(0) + 1)
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("op", ("rmsnorm", "layernorm", "fused_add_rms_norm"))
+@pytest.mark.parametrize("rows,cols", [(256, 3), (256, 257), (256, 512), (257, 512)])
+def test_norm_column_sums_of_infinities(op, rows, cols, dtype):
+    """An infinity or NaN in dy makes its own column's sums what a plain sum makes them,
+    and no other column's, in both programs of the backward (the fp64 reference's sums)."""
+    print(f"\n[gpu-ragged] infinities {op} {rows}x{cols} {dtype}", flush=True)
+    mod = pair_module(op)
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    x, dy, w = rnd(rows, cols), rnd(rows, cols), rnd(cols)
+    bad = [(3, 0, float("inf")), (70, cols - 1, float("-inf")), (200, 1, float("nan"))]
+    if cols > 8:  # both signs in one column; an infinity in the last row and in every row
+        bad += [(5, 4, float("inf")), (69, 4, float("inf")), (rows - 1, 6, float("-inf"))]
+        bad += [(r, 7, float("inf")) for r in range(rows)]
+    for r, c, v in bad:
+        dy[r, c] = v
+    if op == "layernorm" and dtype == torch.float32 and cols > 8:
+        dy[1, 8] = dy[65, 8] = 3e38  # a sum that overflows
+    args, s = [x, w], x.double()
+    if op == "layernorm":
+        args.append(rnd(cols))
+    if op == "fused_add_rms_norm":
+        args.insert(1, rnd(rows, cols))
+        s = s + args[1].double()
+    _, saved = getattr(mod, op + "_forward_with_saved")(*args, 1e-5)
+    grads = getattr(mod, op + "_backward_from_saved")(dy, saved, 1e-5)
+    c = s - s.mean(-1, keepdim=True) if op == "layernorm" else s
+    xhat, gd = c * (c.square().mean(-1, keepdim=True) + 1e-5).rsqrt(), dy.double()
+    sums = [(grads[2 if op == "fused_add_rms_norm" else 1], gd * xhat)]
+    if op == "layernorm":
+        sums.append((grads[2], gd))
+    for got, terms in sums:
+        want = terms.sum(0)
+        if want.numel() > 8:  # the overflowing column of dweight depends on the order
+            got, want, terms = (torch.cat((t[..., :8], t[..., 9:]), -1) for t in (got, want, terms))
+        special = ~torch.isfinite(want)
+        assert special.any()
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(got[special]), kind(want[special]))
+        _close(got[~special], want[~special], dtype, terms.abs().sum(0)[~special] + 1)
+    if op == "layernorm" and dtype == torch.float32 and cols > 8:
+        assert torch.isposinf(grads[2][8])
