@@ -299,23 +299,25 @@ int zero_fill(void* p, size_t bytes, hipStream_t st, const char* what);
 // stride ldr; added in fp32 before c is rounded); r == c with ldr == ldc
 // accumulates in place. With a workspace of at least gemm_workspace_bytes(m, n, k)
 // a product of few output tiles splits k (fp32 partials, a fixed-order sum). splits > 0
-// fixes the k ranges of a 16-bit product whatever its row count (1: none; workspace
-// splits x m x n x 4 bytes); gemm_plan_splits is the choice for a shape.
-int gemm_plan_splits(int64_t m, int64_t n, int64_t k);
+// fixes the k ranges whatever the row count (1: none; workspace splits x m x n x 4 bytes);
+// gemm_plan_splits is the choice for a shape. plan_rows > 0: the product is some of the
+// rows of one of plan_rows rows, and its sums take the order they have there.
+int gemm_plan_splits(int64_t m, int64_t n, int64_t k, int dtype);
 size_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int gemm_launch(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k,
                 int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
                 int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
                 const void* r = nullptr, int64_t ldr = 0, bool r_f32 = false,
-                void* ws = nullptr, size_t ws_bytes = 0, int splits = 0);
+                void* ws = nullptr, size_t ws_bytes = 0, int splits = 0, int64_t plan_rows = 0);
 
 // The fp32 product behind gemm_launch (gemm_f32.hip): arguments as gemm_launch's, already
 // validated; a workspace of gemm_f32_workspace_bytes lets a small output split k.
+int gemm_f32_splits(int64_t m, int64_t n, int64_t k);
 size_t gemm_f32_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int gemm_f32_launch(const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k,
                     int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
                     int64_t b_rows, hipStream_t st, const char* name, const float* r, int64_t ldr,
-                    void* ws, size_t ws_bytes);
+                    void* ws, size_t ws_bytes, int splits, int64_t plan_rows);
 
 // The logits product of the fused linear cross entropy with its softmax terms
 // formed in the epilogue (gemm_kernel.hpp), 16-bit operands only: for logits = x w^T

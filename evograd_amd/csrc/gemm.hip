@@ -69,8 +69,8 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int max_splits, int fixed_sp
   }
   return best;
 }
-int gemm_plan_splits(int64_t M, int64_t N, int64_t K) {
-  return gemm_plan(M, N, K, kMaxSplits, 0).splits;
+int gemm_plan_splits(int64_t M, int64_t N, int64_t K, int dtype) {
+  return dtype == EG_F32 ? gemm_f32_splits(M, N, K) : gemm_plan(M, N, K, kMaxSplits, 0).splits;
 }
 
 // Split tail: a product of more than one wave of tiles (kSplitTarget workgroups per
@@ -117,17 +117,18 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
               int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
               int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
               const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int fixed_splits,
-              const SegArgs& seg);
+              int64_t plan_rows, const SegArgs& seg);
 }  // namespace
 
 int gemm_launch(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                 int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
                 int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
-                const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int splits) {
+                const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int splits,
+                int64_t plan_rows) {
   SegArgs none{};
   none.dim = kSegNone;
   return gemm_impl(A, B, C, M, N, K, lda, ldb, ldc, a_kc, b_kc, a_rows, b_rows, dtype, c_dtype, st,
-                   name, R, ldr, r_f32, ws, ws_bytes, splits, none);
+                   name, R, ldr, r_f32, ws, ws_bytes, splits, plan_rows, none);
 }
 
 namespace {
@@ -135,7 +136,7 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
               int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
               int64_t b_rows, int dtype, int c_dtype, hipStream_t st, const char* name,
               const void* R, int64_t ldr, bool r_f32, void* ws, size_t ws_bytes, int fixed_splits,
-              const SegArgs& seg) {
+              int64_t plan_rows, const SegArgs& seg) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0) {
     set_error("%s: K must be positive", name);
@@ -162,7 +163,7 @@ int gemm_impl(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
     }
     return gemm_f32_launch((const float*)A, (const float*)B, (float*)C, M, N, K, lda, ldb, ldc,
                            a_kc, b_kc, a_rows, b_rows, st, name, (const float*)R, ldr, ws,
-                           ws_bytes);
+                           ws_bytes, fixed_splits, plan_rows);
   }
   if (dtype != EG_BF16 && dtype != EG_F16) {
     set_error("%s: operands must be fp32, bf16 or fp16", name);
@@ -464,5 +465,5 @@ extern "C" int eg_gemm_segmented(const void* a, const void* b, void* c, int64_t 
   if (m == 0 || n == 0) return 0;
   return gemm_impl(pa, pb, pc, m, n, k, lda, ldb, ldc, akc, bkc, akc ? m : k, bkc ? n : k, dtype,
                    c_dtype, as_stream(stream), name, nullptr, 0, false, workspace,
-                   workspace_bytes, 0, g);
+                   workspace_bytes, 0, 0, g);
 }

@@ -205,6 +205,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, floa
 }
 
 // Tiling of an M x N x K product (see the file comment) and its k split over workgroups.
+// Both wide tilings add k in the same order, one chain of MFMAs per output; the 32-wide one
+// and each split have orders of their own.
 constexpr int64_t kF32Tiles = 256, kF32MaxSplits = 8, kF32MinSteps = 8;
 struct F32Plan {
   int64_t tile, tiles, splits;
@@ -221,10 +223,22 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
   return {32, nt, (nk + per - 1) / per};
 }
 
+// The tiling of M rows of a product of `rows` rows, with the whole product's order of sums:
+// its k split, and its 32-wide tiles or the wide ones that suit M.
+F32Plan f32_plan_rows(int64_t M, int64_t rows, int64_t N, int64_t K) {
+  F32Plan p = f32_plan(rows, N, K);
+  auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
+  if (p.tile == 128 && tiles(128) < kF32Tiles) p.tile = 64;
+  p.tiles = tiles(p.tile);
+  return p;
+}
+
 }  // namespace
 }  // namespace gk
 
 using namespace gk;
+
+int gemm_f32_splits(int64_t M, int64_t N, int64_t K) { return (int)f32_plan(M, N, K).splits; }
 
 size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -235,9 +249,11 @@ size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 int gemm_f32_launch(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K,
                     int64_t lda, int64_t ldb, int64_t ldc, bool a_kc, bool b_kc, int64_t a_rows,
                     int64_t b_rows, hipStream_t st, const char* name, const float* R, int64_t ldr,
-                    void* ws, size_t ws_bytes) {
-  F32Plan p = f32_plan(M, N, K);
-  if (p.splits > 1 && !(ws && aligned16(ws) && ws_bytes >= gemm_f32_workspace_bytes(M, N, K)))
+                    void* ws, size_t ws_bytes, int splits, int64_t plan_rows) {
+  F32Plan p = f32_plan_rows(M, plan_rows > 0 ? plan_rows : M, N, K);
+  if (splits > 0) p.splits = splits;
+  if (p.splits > 1 &&
+      !(ws && aligned16(ws) && ws_bytes >= (size_t)p.splits * M * N * sizeof(float)))
     p.splits = 1;
   if (p.tiles >= ((int64_t)1 << 24)) {
     set_error("%s: too many tiles", name);

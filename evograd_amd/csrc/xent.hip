@@ -711,17 +711,19 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
   float* logits = (float*)(ws + L.stats);
   char* dl = ws + L.stats + L.logits;
   float* acc = L.acc ? (float*)(dl + L.dl) : nullptr;
-  // k ranges of the dx product (16-bit inputs): its choice for all rows at once, as far as
-  // dW holds the partials of that many rows, so that dx does not depend on the chunking.
+  // k ranges of the dx product: its choice for all rows at once, as far as the scratch holds
+  // the partials of that many rows (16-bit inputs: dW) or of each row (fp32 inputs: the row's
+  // logits), so that dx does not depend on the chunking. For the same reason the fp32
+  // logits and dx products of a chunk add in the order of the product of all rows.
   // bf16 [1024, 4096, 128256], 64 output tiles on 256 CUs: the product 2708 -> 814 + 13 us.
   const size_t dw_bytes = (size_t)vocab * hidden * es;
-  int dx_splits = 0;
-  if (dtype != EG_F32) {
-    const int64_t fit = (int64_t)(dw_bytes / ((size_t)rows * hidden * sizeof(float)));
-    const int64_t nk = L.vp / 64, s = std::min<int64_t>(fit, gemm_plan_splits(rows, hidden, L.vp));
-    const int64_t per = s > 1 ? (nk + s - 1) / s : nk;
-    dx_splits = (int)((nk + per - 1) / per);
-  }
+  const bool f32 = dtype == EG_F32;
+  const int64_t fit = f32 ? vocab / hidden
+                          : (int64_t)(dw_bytes / ((size_t)rows * hidden * sizeof(float)));
+  const int64_t nk = f32 ? (vocab + 31) / 32 : L.vp / 64;
+  const int64_t want = std::min<int64_t>(fit, gemm_plan_splits(rows, hidden, L.vp, dtype));
+  const int64_t per = want > 1 ? (nk + want - 1) / want : nk;
+  const int dx_splits = (int)((nk + per - 1) / per);
   return dispatch_type(dtype, name, [&](auto tag) {
     using T = decltype(tag);
     T* dlp = (T*)dl;
@@ -761,7 +763,8 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
         if (int rc = check_launch(name)) return rc;
       } else {
         if (int rc = gemm_launch(xc, weight, logits, n, vocab, hidden, hidden, hidden, vocab, true,
-                                 true, n, vocab, dtype, EG_F32, st, name))
+                                 true, n, vocab, dtype, EG_F32, st, name, nullptr, 0, false,
+                                 nullptr, 0, 0, rows))
           return rc;
         const float* none = nullptr;
         if (vocab % 4 == 0) {
@@ -788,13 +791,12 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
       // which the last chunk's dW product writes after its dx product (16-bit inputs;
       // earlier chunks sum in acc), or the chunk's spent logits (fp32 inputs, whose dW
       // product may split as well).
-      const bool f32 = dtype == EG_F32;
       void* spent = f32 ? (void*)logits : nullptr;
       const size_t spent_bytes = f32 ? L.logits : 0;
       if (int rc = gemm_launch(dlp, weight, (T*)dx + r0 * hidden, n, hidden, L.vp, L.vp, hidden,
                                hidden, true, false, n, vocab, dtype, dtype, st, name, nullptr, 0,
                                false, f32 ? spent : dweight, f32 ? spent_bytes : dw_bytes,
-                               dx_splits))
+                               dx_splits, rows))
         return rc;
       // dW = sum over chunks of dl_c^T x_c: into dW directly (one chunk, or fp32
       // inputs), else into the fp32 sum, the last chunk rounding it once into dW

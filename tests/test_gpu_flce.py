@@ -277,3 +277,43 @@ def test_flce_fixup_row_width_edges(vocab, dtype):
     assert bool(((dx.float() - 1.5 * rgx).abs() <= bound_x + 1e-12).all())
     assert bool(((dw.float() - 1.5 * rgw).abs() <= bound_w + 1e-12).all())
     assert torch.equal(dx[2], torch.zeros_like(dx[2]))  # the ignored row
+
+
+# (plan of the logits product, of the dx product): 64-wide tiles and 7 k ranges; 3 ranges, as
+# many as the logits hold; 128-wide tiles and 2 ranges
+@pytest.mark.parametrize("rows,hidden,vocab", [(300, 256, 4096), (300, 256, 1001),
+                                               (1100, 64, 4100)])
+def test_flce_fp32_dx_does_not_depend_on_the_chunking(rows, hidden, vocab):
+    """fp32 inputs: loss and dx of 64-row chunks (the last one ragged) are the bits of one
+    chunk; dweight is the same sum over the rows in another order."""
+    mod = pair_module("fused_linear_cross_entropy")
+    w = Workload(dims=dict(rows=rows, hidden=hidden, vocab=vocab), dtype="float32",
+                 extra={"ignore_every": 7})
+    _note("chunking", w.dims, w.dtype)
+    inp = make_case_inputs(OP, w, "cuda")
+    args = (inp["x"], inp["weight"], inp["target"])
+    runs = []
+    old = mod.CHUNK_ELEMS
+    try:
+        for mod.CHUNK_ELEMS in (old, 64 * vocab):
+            loss, saved = mod.fused_linear_cross_entropy_forward_with_saved(*args)
+            runs.append((loss, *mod.fused_linear_cross_entropy_backward_from_saved(inp["dloss"],
+                                                                                   saved)))
+    finally:
+        mod.CHUNK_ELEMS = old
+    one, many = runs
+    assert torch.equal(one[0], many[0]) and torch.equal(one[1], many[1])
+    # Bound: a logit is off by hidden + 2 roundings of its terms' sum, so a probability by
+    # twice that (its own and the row sum's), relative; then one rounding per term of the
+    # gradient's sum and some for exp, scale and copy.
+    x, wt, t = inp["x"].double(), inp["weight"].double(), inp["target"]
+    ok = t != -100
+    d = torch.softmax(x @ wt.t(), -1).scatter_add(1, t.clamp(min=0)[:, None],
+                                                  torch.ones(rows, 1, device="cuda").double())
+    d = d * ok[:, None] * float(inp["dloss"]) / ok.sum()
+    logit = (hidden + 2) * 2.0 ** -24 * (x.abs() @ wt.abs().t()).max()
+    ref = _ref64(inp)[1:]
+    for run in runs:
+        for got, want, terms, n in ((run[1], ref[0], d @ wt.abs(), vocab),
+                                    (run[2], ref[1], d.t() @ x.abs(), rows)):
+            assert ((got.double() - want).abs() <= ((n + 40) * 2.0 ** -24 + 2 * logit) * terms).all()
