@@ -1116,16 +1116,25 @@ int launch_bwd_small(const T* dy, const T* x, const T* res, const T* w, const fl
 // and its column sum at every width measured (bf16, hidden 1024 / 4096 / 8192, backward call,
 // ring against one launch: RMSNorm 64 rows 9.6 / 11.0 / 10.8 -> 6.2 / 7.2 / 9.9 us, 256 rows
 // 10.2 / 11.9 / 13.6 -> 7.1 / 8.6 / 12.8; LayerNorm 256 rows 10.4 / 13.1 / 17.2 -> 8.5 / 9.9 /
-// 12.8; narrow widths win up to about 500 rows). Its workgroups read rows that others write
-// dx for, so dx must not overlap dy, x or res; where it does the ring runs.
+// 12.8; narrow widths win up to about 500 rows). Its workgroups read what others write
+// outputs for, so no output may overlap an input; where one does the ring runs, which reads a
+// row of dy, x and res before it writes the row's dx, and writes dweight and dbias last.
 constexpr int64_t kSmallRows = 256;
-bool use_bwd_small(int64_t rows, int64_t hidden, size_t elem, const void* dx,
-                   std::initializer_list<const void*> read) {
+bool use_bwd_small(int64_t rows, int64_t hidden, size_t elem, const void* dx, const void* dweight,
+                   const void* dbias, std::initializer_list<const void*> row_inputs,
+                   const void* w, const float* mean, const float* rstd) {
   if (rows > kSmallRows) return false;
-  const uintptr_t n = (uintptr_t)(rows * hidden) * elem, d = (uintptr_t)dx;
-  for (const void* p : read)
-    if (p && (uintptr_t)p < d + n && d < (uintptr_t)p + n) return false;
-  return true;
+  const size_t all = (size_t)(rows * hidden) * elem, row = (size_t)hidden * elem;
+  auto apart = [](const void* a, size_t na, const void* b, size_t nb) {
+    return !a || !b || (uintptr_t)a + na <= (uintptr_t)b || (uintptr_t)b + nb <= (uintptr_t)a;
+  };
+  auto clear = [&](const void* out, size_t n) {
+    for (const void* p : row_inputs)
+      if (!apart(out, n, p, all)) return false;
+    return apart(out, n, w, row) && apart(out, n, mean, rows * sizeof(float)) &&
+           apart(out, n, rstd, rows * sizeof(float));
+  };
+  return clear(dx, all) && clear(dweight, row) && clear(dbias, row);
 }
 
 // Partial rows of the backward (must match the launch). vec: 16-byte packs of elem-byte
@@ -1243,7 +1252,8 @@ static int rms_bwd_impl(const char* name, const void* dy, const void* x, const v
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
     float* part = (float*)workspace;
-    if (use_bwd_small(rows, hidden, sizeof(T), dx, {dy, x, r}))
+    if (use_bwd_small(rows, hidden, sizeof(T), dx, dweight, nullptr, {dy, x, r}, weight, nullptr,
+                      rstd))
       return launch_bwd_small<T, false, ADD>((const T*)dy, (const T*)x, (const T*)r,
                                              (const T*)weight, nullptr, rstd, (T*)dx, (T*)dweight,
                                              nullptr, rows, h, st, name);
@@ -1359,7 +1369,7 @@ extern "C" int eg_layernorm_bwd(const void* dy, const void* x, const void* weigh
     using T = scalar_t;
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
-    if (use_bwd_small(rows, hidden, sizeof(T), dx, {dy, x}))
+    if (use_bwd_small(rows, hidden, sizeof(T), dx, dweight, dbias, {dy, x}, weight, mean, rstd))
       return launch_bwd_small<T, true, false>((const T*)dy, (const T*)x, (const T*)nullptr,
                                               (const T*)weight, mean, rstd, (T*)dx, (T*)dweight,
                                               (T*)dbias, rows, h, st, "eg_layernorm_bwd");

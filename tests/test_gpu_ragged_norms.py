@@ -8,7 +8,7 @@ fp32 bound is the declarations' 1e-5, relative to the row's or column's scale.""
 import pytest
 import torch
 
-from evograd_amd import pair_module
+from evograd_amd import _lib, pair_module
 
 pytestmark = pytest.mark.gpu
 ULP = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
@@ -104,3 +104,36 @@ def test_norm_column_sums_of_infinities(op, rows, cols, dtype):
         _close(got[~special], want[~special], dtype, terms.abs().sum(0)[~special] + 1)
     if op == "layernorm" and dtype == torch.float32 and cols > 8:
         assert torch.isposinf(grads[2][8])
+
+
+@pytest.mark.parametrize("op", ("rmsnorm", "layernorm", "fused_add_rms_norm"))
+@pytest.mark.parametrize("at", ("dx on dy", "dx on x", "dweight on weight"))
+def test_norm_backward_in_place(op, at):
+    """Outputs laid over inputs that the ring has read by then give what separate buffers
+    give (two bf16 roundings of close fp32 sums) at a row count of the one launch, whose
+    workgroups would read what others wrote."""
+    print(f"\n[gpu-ragged] in place {op} {at}", flush=True)
+    rows, cols = 200, 4096
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()
+    entry = {"rmsnorm": "eg_rmsnorm_bwd", "layernorm": "eg_layernorm_bwd",
+             "fused_add_rms_norm": "eg_fused_add_rmsnorm_bwd"}[op]
+    dy, x, r, w = rnd(rows, cols), rnd(rows, cols), rnd(rows, cols), rnd(cols)
+    stats = torch.rand(2, rows, device="cuda", generator=g) + 0.5
+    ws = torch.empty(_lib.query("eg_layernorm_workspace_bytes", rows, cols), dtype=torch.uint8,
+                     device="cuda")
+
+    def run(alias):
+        t = dict(dy=dy.clone(), x=x.clone(), w=w.clone())
+        o = dict(dx=torch.empty_like(x), dw=torch.empty_like(w), db=torch.empty_like(w))
+        if alias:
+            o[{"dx": "dx", "dweight": "dw"}[at.split()[0]]] = t[at.split()[2].replace("weight", "w")]
+        args = [t["dy"], t["x"]] + ([r] if op == "fused_add_rms_norm" else []) + [t["w"]]
+        args += [stats[0], stats[1]] if op == "layernorm" else [stats[1]]
+        args += [o["dx"], o["dw"]] + ([o["db"]] if op == "layernorm" else []) + [ws]
+        _lib.call(entry, *(a.data_ptr() for a in args), rows, cols, _lib.EG_BF16,
+                  _lib.stream_of(x))
+        return [o["dx"], o["dw"]] + ([o["db"]] if op == "layernorm" else [])
+
+    for got, want in zip(run(True), run(False)):
+        torch.testing.assert_close(got, want, rtol=2.0 ** -7, atol=1e-4)
