@@ -718,8 +718,12 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
   // bf16 [1024, 4096, 128256], 64 output tiles on 256 CUs: the product 2708 -> 814 + 13 us.
   const size_t dw_bytes = (size_t)vocab * hidden * es;
   const bool f32 = dtype == EG_F32;
-  const int64_t fit = f32 ? vocab / hidden
-                          : (int64_t)(dw_bytes / ((size_t)rows * hidden * sizeof(float)));
+  // dW laid over the weight is no scratch: the dx product reads the weight.
+  const bool dw_free = (uintptr_t)dweight + dw_bytes <= (uintptr_t)weight ||
+                       (uintptr_t)weight + dw_bytes <= (uintptr_t)dweight;
+  const int64_t fit = f32       ? vocab / hidden
+                      : dw_free ? (int64_t)(dw_bytes / ((size_t)rows * hidden * sizeof(float)))
+                                : 0;
   const int64_t nk = f32 ? (vocab + 31) / 32 : L.vp / 64;
   const int64_t want = std::min<int64_t>(fit, gemm_plan_splits(rows, hidden, L.vp, dtype));
   const int64_t per = want > 1 ? (nk + want - 1) / want : nk;
@@ -795,8 +799,8 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
       const size_t spent_bytes = f32 ? L.logits : 0;
       if (int rc = gemm_launch(dlp, weight, (T*)dx + r0 * hidden, n, hidden, L.vp, L.vp, hidden,
                                hidden, true, false, n, vocab, dtype, dtype, st, name, nullptr, 0,
-                               false, f32 ? spent : dweight, f32 ? spent_bytes : dw_bytes,
-                               dx_splits, rows))
+                               false, f32 ? spent : (dw_free ? dweight : nullptr),
+                               f32 ? spent_bytes : dw_bytes, dx_splits, rows))
         return rc;
       // dW = sum over chunks of dl_c^T x_c: into dW directly (one chunk, or fp32
       // inputs), else into the fp32 sum, the last chunk rounding it once into dW

@@ -339,7 +339,7 @@ int eg_cross_entropy_mean(const int64_t* target, const float* rowloss, void* los
  * target int64 [rows]; a target outside [0, vocab) that is not ignore_index
  * gives NaN. 16-bit inputs need hidden % 64 == 0. The backward scales dx and
  * dweight by dloss / n_valid (eg_scale_copy). dweight's memory also serves as scratch
- * before it is written. */
+ * before it is written, unless it overlaps weight. */
 size_t eg_flce_workspace_bytes(int64_t rows, int64_t hidden, int64_t vocab, int64_t chunk_rows,
                                int dtype);
 int eg_flce_fwd(const void* x, const void* weight, const int64_t* target, float* loss, void* dx,

@@ -13,7 +13,7 @@ import sys
 import pytest
 import torch
 
-from evograd_amd import decls, pair_module
+from evograd_amd import _lib, decls, pair_module
 from evograd_amd.bind import bind
 from evograd_amd.inputs import make_case_inputs
 from evograd_amd.opdecl import Workload
@@ -317,3 +317,31 @@ def test_flce_fp32_dx_does_not_depend_on_the_chunking(rows, hidden, vocab):
         for got, want, terms, n in ((run[1], ref[0], d @ wt.abs(), vocab),
                                     (run[2], ref[1], d.t() @ x.abs(), rows)):
             assert ((got.double() - want).abs() <= ((n + 40) * 2.0 ** -24 + 2 * logit) * terms).all()
+
+
+def test_flce_dweight_over_the_weight():
+    """dweight may take the weight's place in a single chunk (the weight is read before it is
+    written): a shape whose dx product would keep its partials in dweight's memory."""
+    rows, hidden, vocab = 64, 256, 8192
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(rows, hidden, device="cuda", generator=g).bfloat16()
+    wt = (torch.randn(vocab, hidden, device="cuda", generator=g) * hidden ** -0.5).bfloat16()
+    t = torch.randint(0, vocab, (rows,), device="cuda", generator=g)
+    ws = torch.empty(_lib.query("eg_flce_workspace_bytes", rows, hidden, vocab, 0, _lib.EG_BF16),
+                     dtype=torch.uint8, device="cuda")
+    runs = []
+    for alias in (False, True):
+        _note("dweight over weight", alias)
+        w = wt.clone()
+        dw, dx = w if alias else torch.empty_like(w), torch.empty_like(x)
+        loss, n = torch.empty(2, device="cuda").unbind()
+        _lib.call("eg_flce_fwd", x.data_ptr(), w.data_ptr(), t.data_ptr(), loss.data_ptr(),
+                  dx.data_ptr(), dw.data_ptr(), n.data_ptr(), ws.data_ptr(), rows, hidden, vocab,
+                  -100, 0, _lib.EG_BF16, _lib.stream_of(x))
+        runs.append((loss, dx, dw))
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][2], runs[1][2])
+    # dx: the same products summed in other k ranges in fp32, rounded once
+    terms = torch.softmax(x.double() @ wt.double().t(), -1).scatter_add(
+        1, t[:, None], torch.ones(rows, 1, device="cuda").double()) @ wt.double().abs()
+    diff = (runs[0][1].double() - runs[1][1].double()).abs()
+    assert (diff <= 2.0 ** -7 * runs[0][1].double().abs() + vocab * 2.0 ** -23 * terms).all()
