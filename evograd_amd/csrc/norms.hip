@@ -1113,17 +1113,36 @@ int launch_bwd_small(const T* dy, const T* x, const T* res, const T* w, const fl
 }
 
 // The backward entry points take it up to kSmallRows rows, where one launch beats the ring
-// and its column sum at every width measured (bf16, hidden 1024 / 4096 / 8192, backward call,
-// ring against one launch: RMSNorm 64 rows 9.6 / 11.0 / 10.8 -> 6.2 / 7.2 / 9.9 us, 256 rows
-// 10.2 / 11.9 / 13.6 -> 7.1 / 8.6 / 12.8; LayerNorm 256 rows 10.4 / 13.1 / 17.2 -> 8.5 / 9.9 /
-// 12.8; narrow widths win up to about 500 rows). Its workgroups read what others write
+// and its column sum at nearly every width, timed from 1 to 640 rows and 128 to 65536 columns
+// (ring -> one launch, us with cold caches; with the inputs in cache the gain is larger):
+//   bf16 RMSNorm    64 rows, hidden 1024 / 4096 / 8192: 10.0 / 11.4 / 11.1 -> 6.3 / 7.4 / 10.3,
+//                   256 rows: 10.6 / 12.2 / 13.9 -> 7.5 / 9.2 / 12.9
+//   bf16 LayerNorm  256 rows, 1024 / 4096 / 16384: 10.8 / 13.4 / 46.3 -> 8.5 / 10.1 / 20.4
+//   bf16 residual   256 rows, 1024 / 4096 / 8192: 10.6 / 13.1 / 15.4 -> 8.4 / 10.4 / 15.5
+//   fp32 RMSNorm    256 rows, 1024 / 4096 / 8192: 10.1 / 11.2 / 16.2 -> 7.2 / 10.7 / 15.9
+//   past 2048 packs, where the ring's registers spill: bf16 RMSNorm [256, 32768] 103 -> 36.
+// In the ring's two-pack configuration of 1024 threads (1025-2048 packs) the ring reads its
+// inputs once, which wins at the wide end (kSmallPacksMax) in two cases, cold and cached alike:
+// 16-bit RMSNorm of few rows (bf16 [1, 16384] 11.6 -> 14.1, [32, 16384] 13.2 -> 14.8, [16, 14336]
+// 12.7 -> 13.1; at [1, 12288] and [64, 16384] cached times are equal, at [64, 14336] one launch is
+// 1.13x ahead) and the fp32 residual form of many (three inputs read twice: [256, 8192] 19.0 ->
+// 20.6, [256, 7168] 17.5 -> 18.8; [200, 8192] 18.0 -> 18.1, cached 1.07x ahead). Past kSmallRows the gain depends on width
+// and form (384 rows: bf16 RMSNorm 4096 12.7 -> 11.0, residual 8192 16.2 -> 20.5; 512 rows: bf16
+// RMSNorm 2048 12.2 -> 10.4, 4096 13.0 -> 13.7), so the ring takes every such call.
+//
+// Its workgroups read what others write
 // outputs for, so no output may overlap an input; where one does the ring runs, which reads a
 // row of dy, x and res before it writes the row's dx, and writes dweight and dbias last.
-constexpr int64_t kSmallRows = 256;
-bool use_bwd_small(int64_t rows, int64_t hidden, size_t elem, const void* dx, const void* dweight,
-                   const void* dbias, std::initializer_list<const void*> row_inputs,
-                   const void* w, const float* mean, const float* rstd) {
+constexpr int64_t kSmallRows = 256, kSmallPacksMax = 1536;
+bool use_bwd_small(int64_t rows, int64_t hidden, size_t elem, bool ln, bool add, const void* dx,
+                   const void* dweight, const void* dbias,
+                   std::initializer_list<const void*> row_inputs, const void* w,
+                   const float* mean, const float* rstd) {
   if (rows > kSmallRows) return false;
+  const int64_t packs = (hidden * (int64_t)elem + 15) / 16;
+  if (packs > kSmallPacksMax && packs <= 2048 &&
+      ((!ln && !add && elem == 2 && rows <= 32) || (add && elem == 4 && rows > 224)))
+    return false;
   const size_t all = (size_t)(rows * hidden) * elem, row = (size_t)hidden * elem;
   auto apart = [](const void* a, size_t na, const void* b, size_t nb) {
     return !a || !b || (uintptr_t)a + na <= (uintptr_t)b || (uintptr_t)b + nb <= (uintptr_t)a;
@@ -1252,8 +1271,8 @@ static int rms_bwd_impl(const char* name, const void* dy, const void* x, const v
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
     float* part = (float*)workspace;
-    if (use_bwd_small(rows, hidden, sizeof(T), dx, dweight, nullptr, {dy, x, r}, weight, nullptr,
-                      rstd))
+    if (use_bwd_small(rows, hidden, sizeof(T), false, ADD, dx, dweight, nullptr, {dy, x, r},
+                      weight, nullptr, rstd))
       return launch_bwd_small<T, false, ADD>((const T*)dy, (const T*)x, (const T*)r,
                                              (const T*)weight, nullptr, rstd, (T*)dx, (T*)dweight,
                                              nullptr, rows, h, st, name);
@@ -1369,7 +1388,8 @@ extern "C" int eg_layernorm_bwd(const void* dy, const void* x, const void* weigh
     using T = scalar_t;
     constexpr int V = 16 / sizeof(T);
     const int h = (int)hidden;
-    if (use_bwd_small(rows, hidden, sizeof(T), dx, dweight, dbias, {dy, x}, weight, mean, rstd))
+    if (use_bwd_small(rows, hidden, sizeof(T), true, false, dx, dweight, dbias, {dy, x}, weight,
+                      mean, rstd))
       return launch_bwd_small<T, true, false>((const T*)dy, (const T*)x, (const T*)nullptr,
                                               (const T*)weight, mean, rstd, (T*)dx, (T*)dweight,
                                               (T*)dbias, rows, h, st, "eg_layernorm_bwd");

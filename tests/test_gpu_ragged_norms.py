@@ -137,3 +137,12 @@ def test_norm_backward_in_place(op, at):
 
     for got, want in zip(run(True), run(False)):
         torch.testing.assert_close(got, want, rtol=2.0 ** -7, atol=1e-4)
+
+
+@pytest.mark.parametrize("op,rows,cols,dtype", [
+    ("rmsnorm", 32, 12296, torch.bfloat16), ("rmsnorm", 33, 12296, torch.bfloat16),
+    ("rmsnorm", 4, 16384, torch.float16), ("fused_add_rms_norm", 225, 6148, torch.float32),
+    ("fused_add_rms_norm", 224, 8192, torch.float32), ("layernorm", 3, 16384, torch.bfloat16)])
+def test_norms_wide_rows_on_either_program(op, rows, cols, dtype):
+    """Both sides of the lines between the two backward programs at 1537-2048 packs."""
+    test_norms_ragged_rows(op, rows, cols, 0, dtype)
