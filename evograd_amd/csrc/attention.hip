@@ -1088,7 +1088,7 @@ int dkdv_parts(int64_t BHkv, int64_t S, int64_t D) {
   if (wgs <= 0 || wgs >= kDkdvTarget) return 1;
   return (int)std::min<int64_t>(kDkdvMaxParts, (kDkdvTarget + wgs - 1) / wgs);
 }
-// Parts to take, up to that bound (which sizes the workspace): each shortens the longest
+// Parts to take, up to that bound: each shortens the longest
 // walk until the chip is full (two workgroups per CU) and costs its slabs' write and read.
 // In us, 1.1 (D = 128) or 0.9 (64) per 32-row step, 1.6 per million elements of dK and
 // part, and 5 for the reduction: fitted over 48 shapes timed at every number of parts; the
@@ -1112,8 +1112,8 @@ int dkdv_split(int64_t BHkv, int64_t group, int64_t S, int64_t D) {
 // Backward workspace after delta (fp32 [BH, S], rounded up to 256 bytes): the split
 // walk's slabs, 2 x parts x BHkv x S x D fp32 (none without a split).
 size_t attn_delta_bytes(int64_t BH, int64_t S) { return ((size_t)(BH * S) * 4 + 255) / 256 * 256; }
-size_t attn_part_bytes(int64_t BHkv, int64_t S, int64_t D) {
-  const int parts = dkdv_parts(BHkv, S, D);
+size_t attn_part_bytes(int64_t BHkv, int64_t group, int64_t S, int64_t D) {
+  const int parts = dkdv_split(BHkv, group, S, D);
   return parts > 1 ? (size_t)2 * parts * BHkv * S * D * 4 : 0;
 }
 
@@ -1286,7 +1286,7 @@ extern "C" size_t eg_attn_gqa_workspace_bytes(int64_t batch, int64_t heads, int6
   if (batch <= 0 || heads <= 0 || seq <= 0 || kv_heads <= 0) return 0;
   // the dtype is not known here: the larger of the MFMA and the generic kernels' slabs
   return attn_delta_bytes(batch * heads, seq) +
-         std::max(attn_part_bytes(batch * kv_heads, seq, head_dim),
+         std::max(attn_part_bytes(batch * kv_heads, heads / kv_heads, seq, head_dim),
                   attn_generic_part_bytes(batch, heads, kv_heads, seq, head_dim));
 }
 
@@ -1380,7 +1380,8 @@ extern "C" size_t eg_llama3_attn_workspace_bytes(int64_t batch, int64_t heads, i
                                                  int64_t seq, int64_t head_dim) {
   if (batch <= 0 || heads <= 0 || kv_heads <= 0 || seq <= 0 || head_dim <= 0) return 0;
   return llama3_ws_qr(batch, heads, seq, head_dim) + llama3_ws_kr(batch, kv_heads, seq, head_dim) +
-         attn_delta_bytes(batch * heads, seq) + attn_part_bytes(batch * kv_heads, seq, head_dim);
+         attn_delta_bytes(batch * heads, seq) +
+         attn_part_bytes(batch * kv_heads, heads / kv_heads, seq, head_dim);
 }
 
 template <typename F>

@@ -228,9 +228,10 @@ int eg_attn_gqa_fwd(const void* q, const void* k, const void* v, void* o, float*
  * heads, seq] (heads = query heads), rounded up to 256 bytes; then, for shapes with
  * fewer than 1024 (kv head, 128-key block) pairs, where the dK/dV walk over the
  * query tiles may be split into parts (a choice of the shape alone, at most
- * min(8, ceil(1024 / pairs))), the fp32 sums of that many: 2 x parts x batch x
- * kv_heads x seq x head_dim x 4 bytes (head sizes other than 64 and 128: the same with
- * fewer than 512 pairs of 16-key blocks).
+ * min(8, ceil(1024 / pairs))), the parts' fp32 sums: 2 x parts x batch x kv_heads x seq x
+ * head_dim x 4 bytes, nothing where one part is taken (fp32 tensors and head sizes other
+ * than 64 and 128: the same with fewer than 512 pairs of 16-key blocks; the dtype is not an
+ * argument, so at 64 and 128 the larger of the two).
  * eg_attn_workspace_bytes (for eg_attn_bwd) is this with kv_heads = heads. */
 size_t eg_attn_gqa_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads,
                                    int64_t seq, int64_t head_dim);

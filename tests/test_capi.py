@@ -125,6 +125,24 @@ def test_attention_workspace_holds_the_split_walk_only_when_split():
 
 
 @pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("B,H,KVH,S,D,parts", [
+    (4, 8, 8, 512, 128, 1), (4, 8, 8, 300, 64, 1), (2, 12, 12, 1000, 64, 3),
+    (1, 8, 8, 2048, 128, 5), (1, 8, 8, 1500, 64, 6), (1, 4, 4, 8192, 64, 4),
+    (1, 2, 1, 768, 128, 8), (1, 32, 32, 200, 64, 1), (1, 4, 4, 64, 64, 1)])
+def test_attention_workspace_holds_the_parts_that_are_taken(B, H, KVH, S, D, parts):
+    """Not the most that could be: the slabs of a walk that is not split, or of parts that are
+    not taken, are not allocated."""
+    got = _lib.query("eg_attn_gqa_workspace_bytes", B, H, KVH, S, D) - (B * H * S * 4 + 255) // 256 * 256
+    slab = 2 * B * KVH * S * D * 4
+    # fp32 tensors of the same shape take this many (two workgroups of 16 keys per CU, two
+    # steps for each of a workgroup's four waves)
+    blocks = B * KVH * -(-S // 16)
+    generic = max(1, min(-(-512 // blocks), H // KVH * -(-S // 16) // 8, 8))
+    most = max(parts, generic)
+    assert got == (most * slab if most > 1 else 0)
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
 def test_host_side_validation_errors_without_gpu():
     """Argument errors are reported before any launch (no device needed)."""
     with pytest.raises(RuntimeError, match="negative"):
