@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from evograd_amd import _lib
+from evograd_amd.timing import KernelTimer
 
 pytestmark = pytest.mark.gpu
 
@@ -294,3 +295,74 @@ def test_gemm_segmented_is_the_concatenated_product_bitwise(dim, sizes, mnk, akc
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     assert ((got.double() - ref).abs() <= ulp * ref.abs() + 4e-6 * K).all()
 
+
+
+# ------------------------------------------------------- the 256 x 256 kernel
+# The products above are small enough for the 128 x 128 kernel (tests/test_gpu_gemm_mid.py
+# has its own); these are not, and each checks which kernel ran.
+LARGE = [
+    # more than 128 tiles, unsplit, ragged in M, N and (k-major) K
+    *((2900, 3000, 320, *lay) for lay in LAYOUTS), (2900, 3000, 100, False, False),
+    # split k, ragged likewise
+    *((1000, 4000, 14336, *lay) for lay in LAYOUTS), (700, 3001, 9000, False, False),
+]
+
+
+@pytest.mark.parametrize("dtype,cdt", [(torch.bfloat16, torch.bfloat16),
+                                       (torch.float16, torch.float16),
+                                       (torch.float16, torch.float32)])
+@pytest.mark.parametrize("M,N,K,akc,bkc", LARGE)
+def test_gemm_large_tiles(M, N, K, akc, bkc, dtype, cdt):
+    """Against fp64, with and without a residual: fp32 accumulation of K exact products (at
+    most (K + 20) 2^-24 of the sum of the absolute terms), then one rounding."""
+    print(f"\n[gpu-gemm] large {dtype} -> {cdt} {M}x{N}x{K} akc={akc} bkc={bkc}", flush=True)
+    A, B, a, b, lda, ldb = _operands(M, N, K, akc, bkc, dtype, M + N + K)
+    need = _lib.query("eg_gemm_workspace_bytes", M, N, K, _lib.dtype_tag(dtype))
+    assert (need > 0) == (K > 1000)
+    ws = torch.full((max(need, 16),), 255, dtype=torch.uint8, device="cuda")
+    ldc = _r8(N) + (3 if cdt == torch.float32 else 0)
+    want, terms = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[cdt]
+    timer = KernelTimer()
+    for r in (None, torch.randn(M, ldc, device="cuda").to(cdt)):
+        w, t = (want, terms) if r is None else (want + r[:, :N].double(),
+                                                terms + r[:, :N].double().abs())
+        c = torch.full((M, ldc), float("nan"), device="cuda", dtype=cdt)
+        split = need > 0 and r is not None  # the second call's second launch
+        timer.arm(int(split))
+        _lib.call("eg_gemm", a.data_ptr(), b.data_ptr(), c.data_ptr(), _lib.ptr(r), M, N, K, lda,
+                  ldb, ldc, 0 if r is None else ldc, int(akc), int(bkc), _lib.dtype_tag(dtype),
+                  _lib.dtype_tag(cdt), ws.data_ptr(), need, _lib.stream_of(a))
+        assert timer.label() == ("splitk_reduce_kernel" if split else "gemm_kernel")
+        assert ((c[:, :N].double() - w).abs()
+                <= t * (K + 20) * 2.0 ** -24 + w.abs() * ulp + 2.0 ** -25).all()
+        assert torch.isnan(c[:, N:]).all()
+    timer.close()
+
+
+LARGE_SEGMENTS = [
+    (3, [4096, 1024, 1024], (2048, 4096, None)),  # the decoder layer's q/k/v gradient, 2 parts
+    (3, [128, 64, 192], (2900, 3000, None)),      # more than 128 tiles, unsplit
+    (1, [2048, 2304], (None, 2100, 384)),
+    (1, [256, 644], (None, 4000, 9024)),          # M segments, split k, ragged
+    (2, [2048, 1052], (2900, None, 384)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("dim,sizes,mnk", LARGE_SEGMENTS)
+def test_gemm_large_tiles_segmented(dim, sizes, mnk, akc, bkc, dtype, monkeypatch):
+    timer, ran, call = KernelTimer(), [], _lib.call
+
+    def watched(name, *args):
+        timer.arm(0)
+        call(name, *args)
+        ran.append((name, timer.label()))
+
+    monkeypatch.setattr(_lib, "call", watched)
+    # arming is itself a library call
+    monkeypatch.setattr(timer, "arm", lambda i: call("eg_time_kernel", timer.start, timer.stop, i))
+    test_gemm_segmented_is_the_concatenated_product_bitwise(dim, sizes, mnk, akc, bkc, dtype)
+    assert ran == [("eg_gemm", "gemm_kernel"), ("eg_gemm_segmented", "gemm_kernel")]
+    timer.close()
