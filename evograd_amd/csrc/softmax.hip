@@ -48,7 +48,8 @@ __device__ __forceinline__ void load_row(const T* __restrict__ row, int cols, fl
     for (int it = 0; it < ITEMS; ++it) {
       const int c = (it * BLOCK + (int)threadIdx.x) * VEC;
       if (c < cols) {
-        rowwise::load_pack<T, VEC, NT, RAG>(row, c, cols, fill, v[it]);
+        if constexpr (RAG) load_ragged<T, VEC, NT>(row + ragged_pack<VEC>(c, cols).c, v[it]);
+        else load_vec<T, VEC, NT>(row + c, v[it]);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[it][i] = fill;
@@ -77,9 +78,23 @@ __device__ __forceinline__ void store_row(T* __restrict__ row, int cols,
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int c = (it * BLOCK + (int)threadIdx.x) * VEC;
-      if (c < cols) rowwise::store_pack<T, VEC, NT, RAG>(row, c, cols, v[it]);
+      if (c < cols) {
+        // a ragged row's last pack stores the elements it shares with the one before as well:
+        // both hold the same bits
+        if constexpr (RAG) store_ragged<T, VEC, NT>(row + ragged_pack<VEC>(c, cols).c, 0, v[it]);
+        else store_vec<T, VEC, NT>(row + c, v[it]);
+      }
     }
   }
+}
+
+// Whether element i of this thread's pack `it` counts in the row's sums: in a ragged row's
+// last pack, the elements that are its own.
+template <int VEC, int BLOCK, bool RAG>
+__device__ __forceinline__ bool counts(int it, int i, int cols) {
+  if constexpr (!RAG) return true;
+  const int c = (it * BLOCK + (int)threadIdx.x) * VEC;
+  return i >= c - (cols - VEC) || c >= cols;
 }
 
 template <typename T, int VEC, int ITEMS, int BLOCK, bool NT, bool RAG>
@@ -105,7 +120,7 @@ __global__ __launch_bounds__(BLOCK) void softmax_fwd_reg(const T* __restrict__ x
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       v[it][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[it][i], kL2e, -ml));
-      s += v[it][i];
+      s += counts<VEC, BLOCK, RAG>(it, i, cols) ? v[it][i] : 0.f;
     }
   s = block_reduce<BLOCK>(s, SumOp(), lds);
   const float inv = 1.0f / s;
@@ -129,7 +144,8 @@ __global__ __launch_bounds__(BLOCK) void softmax_bwd_reg(const T* __restrict__ y
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) d += gv[it][i] * yv[it][i];
+    for (int i = 0; i < VEC; ++i)
+      d += counts<VEC, BLOCK, RAG>(it, i, cols) ? gv[it][i] * yv[it][i] : 0.f;
   d = block_reduce<BLOCK>(d, SumOp(), lds);
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
@@ -494,12 +510,23 @@ void softmax_bwd_vec(const T* y, const T* dy, T* dx, int64_t rows, int cols, hip
 
 // Rows that are not whole aligned packs: unaligned 16-byte packs (bf16 [2000, 10007]
 // forward and backward 91.2 -> 49.6 us, fp32 [8000, 1001] 38.2 -> 31.3, [1000, 9001] 44.7 ->
-// 37.2), except fp32 rows of 4097-8192 columns, which one register row of single elements
-// takes at whole cache lines per wave ([2000, 5001] 37.9 us against 39.5, [2000, 8001] 57.2
-// against 64.4), and rows narrower than a pack.
+// 37.2), except
+//   fp32 rows of 4097-8192 columns, which one register row of single elements takes at whole
+//   cache lines per wave ([2000, 5001] 37.9 us against 39.5, [2000, 8001] 57.2 against 64.4);
+//   rows of one wave's elements (16 of 64 lanes would hold a pack; [32768, 33] forward fp32
+//   11.1 against 12.2, bf16 10.5 against 12.2);
+//   few rows, where a launch is latency and single elements save 0.2-0.5 us of it. Forward,
+//   single elements against packs, on both sides of the lines below: fp32 [1024, 201] 3.6 / 3.8
+//   and [4096, 201] 5.8 / 4.8, bf16 [1024, 257] 3.9 / 3.9 and [4096, 257] 5.9 / 4.6, fp32
+//   [512, 1501] 4.1 / 4.9 and [2048, 1501] 7.9 / 7.1, bf16 [256, 3739] 4.2 / 4.6 and [1024, 3739]
+//   8.3 / 6.3; backward fp32 [1024, 1001] 4.0 / 4.6 and [4096, 1001] 10.1 / 8.5, bf16 [512, 3001]
+//   4.5 / 4.6 and [2048, 3001] 14.7 / 9.7.
 template <typename T>
-bool ragged_packs(int64_t cols) {
-  return cols >= (int64_t)(16 / sizeof(T)) && !(sizeof(T) == 4 && cols > 4096 && cols <= 8192);
+bool ragged_packs(int64_t rows, int64_t cols, bool bwd) {
+  if (cols <= kWave || (sizeof(T) == 4 && cols > 4096 && cols <= 8192)) return false;
+  if (cols > 4096) return true;
+  const int64_t from = cols <= 128 ? 16384 : cols <= 512 ? 2048 : cols <= 2048 ? 1024 : 512;
+  return rows >= (bwd ? 2 * from : from);
 }
 
 int check_dims(const char* what, int64_t rows, int64_t cols) {
@@ -534,7 +561,7 @@ extern "C" int eg_softmax_fwd(const void* x, void* y, int64_t rows, int64_t cols
     T* yp = static_cast<T*>(y);
     if (cols % V == 0 && aligned16(x) && aligned16(y))
       softmax_fwd_vec<T, V>(xp, yp, rows, (int)cols, st);
-    else if (ragged_packs<T>(cols))
+    else if (ragged_packs<T>(rows, cols, false))
       softmax_fwd_vec<T, V, true>(xp, yp, rows, (int)cols, st);
     else
       softmax_fwd_vec<T, 1>(xp, yp, rows, (int)cols, st);
@@ -557,7 +584,7 @@ extern "C" int eg_softmax_bwd(const void* y, const void* dy, void* dx, int64_t r
     T* dp = static_cast<T*>(dx);
     if (cols % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx))
       softmax_bwd_vec<T, V>(yp, gp, dp, rows, (int)cols, st);
-    else if (ragged_packs<T>(cols))
+    else if (ragged_packs<T>(rows, cols, true))
       softmax_bwd_vec<T, V, true>(yp, gp, dp, rows, (int)cols, st);
     else
       softmax_bwd_vec<T, 1>(yp, gp, dp, rows, (int)cols, st);

@@ -10,7 +10,7 @@ reads a rounded y), an fp32 one within 1e-5 (the declarations' gate)."""
 import pytest
 import torch
 
-from evograd_amd import pair_module
+from evograd_amd import _lib, pair_module
 
 pytestmark = pytest.mark.gpu
 EPS = {torch.float32: 1e-5, torch.float16: 2.0 ** -9, torch.bfloat16: 2.0 ** -6}
@@ -73,3 +73,36 @@ def test_cross_entropy_ragged_rows(rows, cols, offset, dtype):
     want = torch.exp(x.double() - lse[:, None]).scatter_add(
         1, at, -torch.ones_like(at, dtype=torch.float64)) * (ok[:, None] / n)
     _close(dl, want, dtype, scale=1.0 / (rows * cols))
+
+
+# Row counts on both sides of the lines between single elements and packs, per width.
+LINES = [(16383, 65, 0), (16384, 67, 0), (32768, 127, 0), (2047, 129, 1), (2048, 200, 1),
+         (4095, 511, 0), (4096, 257, 0), (1023, 513, 0), (1024, 1001, 3), (2048, 2047, 0),
+         (511, 2049, 0), (512, 4095, 0), (1024, 2050, 1)]
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("rows,cols,offset", LINES)
+def test_softmax_ragged_rows_many(rows, cols, offset, dtype):
+    test_softmax_ragged_rows(rows, cols, offset, dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+@pytest.mark.parametrize("rows,cols", [(2048, 501), (4096, 501), (1024, 3739), (3, 33333),
+                                       (2, 131075)])
+def test_softmax_ragged_rows_in_place(rows, cols, dtype):
+    """y over x, and dx over dy or over y, give the bits of separate buffers."""
+    print(f"\n[gpu-ragged] softmax in place {rows}x{cols} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(rows, cols, device="cuda", generator=g).to(dtype)
+    dy = torch.randn(rows, cols, device="cuda", generator=g).to(dtype)
+    tail = (rows, cols, _lib.dtype_tag(dtype), _lib.stream_of(x))
+    y, z, dx = torch.empty_like(x), x.clone(), torch.empty_like(x)
+    for a, b in ((x, y), (z, z)):
+        _lib.call("eg_softmax_fwd", a.data_ptr(), b.data_ptr(), *tail)
+    assert torch.equal(y, z)
+    _lib.call("eg_softmax_bwd", y.data_ptr(), dy.data_ptr(), dx.data_ptr(), *tail)
+    over_dy, over_y = dy.clone(), y.clone()
+    _lib.call("eg_softmax_bwd", y.data_ptr(), over_dy.data_ptr(), over_dy.data_ptr(), *tail)
+    _lib.call("eg_softmax_bwd", over_y.data_ptr(), dy.data_ptr(), over_y.data_ptr(), *tail)
+    assert torch.equal(dx, over_dy) and torch.equal(dx, over_y)
