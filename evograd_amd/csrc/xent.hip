@@ -22,9 +22,11 @@
 //   xent_bwd_flat_kernel  one read of the logits and one write of dlogits, workgroups
 //                     in address order over the flattened matrix; dloss read from
 //                     device memory.
+//   xent_bwd_rows_kernel  few narrow rows: one workgroup per row (bwd_flat has the line).
 // Rows that are no multiple of a 16-byte pack are read and written in unaligned packs
-// (eg_common.hpp): bf16 [4096, 50257] forward and backward 677 us element by element, 229
-// so; fp32 backward 1.5x faster at any odd width past 2500.
+// (eg_common.hpp) where that pays (fwd_ragged_packs, bwd_ragged_packs): bf16 [4096, 50257]
+// forward and backward 677 us element by element, 229 so; fp32 backward 1.5x faster at any
+// odd width past 2500.
 //   scale_copy_kernel dst = src * mul / div with a dtype conversion (the fused
 //                     linear cross entropy's dweight conversion and its dloss / n
 //                     scaling).
@@ -49,6 +51,7 @@ using rowwise::kFlatUnroll;
 using rowwise::kLog2e;
 using rowwise::kUnroll;
 using rowwise::pick_row_block;
+constexpr int kBwdBlock = 256;
 constexpr int kMeanBlock = 1024;
 
 template <typename T, int VEC, int BLOCK, bool NT, bool RAG>
@@ -159,19 +162,19 @@ __device__ __forceinline__ void grad_pack(const RowGrad& rg, int c, const float 
 // (b + 1) * kFlatPer) in address order, so the workgroups in flight stream through
 // contiguous memory. With at least kFlatPer packs per row a workgroup spans at most two
 // rows, whose factors every thread holds; with narrower rows (MANY) each pack finds its
-// row by a 32-bit division and takes that row's factors (one workgroup per row instead
-// left most of its threads without a pack: bf16
-// [8000, 1000] 10.3 -> 8.8 us, fp32 [8000, 501] 8.7 -> 7.8).
-// RAG: ragged rows. TI is the logits type, TO the gradient's, TD the type of dloss.
+// row by a 32-bit division and takes that row's factors.
+// RAG: ragged rows; `whole`: dx does not overlap x, so a row's last pack is stored with the
+// elements it shares with the one before (both hold the same bits). TI is the logits type, TO the gradient's, TD the type of dloss.
 template <typename TI, typename TO, typename TD, int VEC, bool NT, bool RAG, bool MANY>
 __global__ __launch_bounds__(kFlatBlock) void xent_bwd_flat_kernel(
     const TD* __restrict__ dloss, const TI* __restrict__ x, const int64_t* __restrict__ target,
     const float* __restrict__ lse, const float* __restrict__ n_valid, TO* __restrict__ dx,
-    int64_t rows, int cols, int64_t ldd, int64_t ignore_index) {
+    int64_t rows, int cols, int64_t ldd, int64_t ignore_index, bool whole) {
   const int64_t ppr = (cols + VEC - 1) / VEC;  // packs per row
   const int64_t npack = rows * ppr;
   const int64_t first = (int64_t)blockIdx.x * kFlatPer;
-  const int64_t row0 = first / ppr;
+  // (a 64-bit division takes several times a 32-bit one's instructions)
+  const int64_t row0 = npack >> 32 ? first / ppr : (unsigned)first / (unsigned)ppr;
   const int64_t at0 = row0 * ppr;
   RowGrad rg[MANY ? kFlatUnroll : 2];
   if constexpr (!MANY) {
@@ -208,11 +211,41 @@ __global__ __launch_bounds__(kFlatBlock) void xent_bwd_flat_kernel(
       if constexpr (MANY) grad_pack<VEC>(rg[u], k.c, v[u], o);
       else grad_pack<VEC>(r ? rg[1] : rg[0], k.c, v[u], o);
       TO* d = dx + (row0 + r) * ldd + k.c;
-      if constexpr (RAG) store_ragged<TO, VEC, NT>(d, k.lo, o);
+      if constexpr (RAG) store_ragged<TO, VEC, NT>(d, whole ? 0 : k.lo, o);
       else store_vec<TO, VEC, NT>(d, o);
     }
   }
 }
+
+// One workgroup per row of at most kBwdBlock * kUnroll packs.
+template <typename TI, typename TO, typename TD, int VEC, bool NT>
+__global__ __launch_bounds__(kBwdBlock) void xent_bwd_rows_kernel(
+    const TD* __restrict__ dloss, const TI* __restrict__ x, const int64_t* __restrict__ target,
+    const float* __restrict__ lse, const float* __restrict__ n_valid, TO* __restrict__ dx,
+    int cols, int64_t ldd, int64_t ignore_index) {
+  constexpr int STEP = kBwdBlock * VEC;
+  const int64_t row = blockIdx.x;
+  const RowGrad rg = row_grad(dloss, target, lse, n_valid, row, cols, ignore_index);
+  const int c0 = (int)threadIdx.x * VEC;
+  const TI* __restrict__ xr = x + row * cols;
+  TO* __restrict__ dr = dx + row * ldd;
+  float v[kUnroll][VEC];
+#pragma unroll
+  for (int u = 0; u < kUnroll; ++u) {
+    const int c = c0 + u * STEP;
+    if (c < cols && !rg.ignored) load_vec<TI, VEC, NT>(xr + c, v[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kUnroll; ++u) {
+    const int c = c0 + u * STEP;
+    if (c < cols) {
+      float o[VEC];
+      grad_pack<VEC>(rg, c, v[u], o);
+      store_vec<TO, VEC, NT>(dr + c, o);
+    }
+  }
+}
+static_assert(kFlatPer <= kBwdBlock * kUnroll, "a row below kFlatPer packs fits its workgroup");
 
 // dst[i] = src[i] * mul[0] / div[0] (either factor optional). Workgroups cover
 // consecutive runs of kScaleUnroll x 256 packs in address order, every load of a
@@ -256,6 +289,18 @@ struct LseLaunch {
   }
 };
 
+// Rows of fewer than kFlatPer packs (of `vec` elements of elem bytes): the flat kernel (MANY),
+// or a workgroup per row. The latter leaves threads without a pack and is launched once per row,
+// the former divides per pack and gathers row factors; us, rows against flat:
+//   [8192, 64] fp32 6.1 / 3.8, bf16 6.7 / 4.1; [8192, 1000] bf16 11.3 / 8.8, fp32 12.4 / 13.0;
+//   [1024, 1000] bf16 4.1 / 4.6, fp32 4.1 / 4.6; [2048, 1536] bf16 5.3 / 6.4, fp32 5.9 / 6.6;
+//   [8192, 3000] fp32 36.0 / 33.4, bf16 19.0 / 20.9; [8192, 4096] bf16 24.2 / 26.5;
+//   in single elements [8192, 1001] fp32 14.4 / 23.5.
+inline bool bwd_flat(int64_t rows, int64_t ppr, int vec, int elem) {
+  return ppr >= kFlatPer ||
+         (rows >= 4096 && (ppr <= 160 || (vec > 1 && elem == 4 && ppr > 400)));
+}
+
 // dlogits rows are written with row stride ldd (>= cols, a multiple of VEC unless RAG).
 template <typename TI, typename TO, typename TD, int VEC, bool RAG = false>
 void launch_bwd(const TD* gp, const TI* xp, const int64_t* target, const float* lse,
@@ -264,13 +309,37 @@ void launch_bwd(const TD* gp, const TI* xp, const int64_t* target, const float* 
   constexpr bool NT = VEC * sizeof(TI) == 16;
   if (ldd < 0) ldd = cols;
   const int64_t ppr = (cols + VEC - 1) / VEC;
+  if constexpr (!RAG)
+    if (!bwd_flat(rows, ppr, VEC, sizeof(TI))) {
+      EG_LAUNCH((xent_bwd_rows_kernel<TI, TO, TD, VEC, NT>), dim3((unsigned)rows),
+                dim3(kBwdBlock), 0, st, gp, xp, target, lse, n_valid, dp, cols, ldd,
+                ignore_index);
+      return;
+    }
   const dim3 grid((unsigned)((rows * ppr + kFlatPer - 1) / kFlatPer));
+  const bool whole = (uintptr_t)(dp + rows * ldd) <= (uintptr_t)xp ||
+                     (uintptr_t)(xp + rows * cols) <= (uintptr_t)dp;
   if (ppr >= kFlatPer)
     EG_LAUNCH((xent_bwd_flat_kernel<TI, TO, TD, VEC, NT, RAG, false>), grid, dim3(kFlatBlock), 0,
-              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index);
+              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index, whole);
   else
     EG_LAUNCH((xent_bwd_flat_kernel<TI, TO, TD, VEC, NT, RAG, true>), grid, dim3(kFlatBlock), 0,
-              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index);
+              st, gp, xp, target, lse, n_valid, dp, rows, cols, ldd, ignore_index, whole);
+}
+
+// Ragged rows in unaligned packs rather than single elements, us (elements / packs).
+// Forward: from 256 columns ([65536, 63] bf16 39.5 / 49.1, fp32 39.9 / 42.2; [65536, 235] 46.4 /
+// 51.1 and 43.7 / 45.6; [32768, 257] 32.1 / 27.5 and 31.4 / 25.8; [512, 257] equal).
+inline bool fwd_ragged_packs(int64_t cols) { return cols >= 256; }
+// Backward: where there is enough of them. Rows that a workgroup's single elements cover
+// (kFlatPer columns): [4096, 301] bf16 5.0 / 5.6, fp32 5.2 / 5.7, [8192, 301] 7.1 / 6.8 and
+// 7.5 / 6.9, fp32 [6001, 1001] 11.5 / 11.0, [32768, 1001] 45.7 / 48.9, [65536, 1001] 107.9 / 93.5.
+// Wider rows: [512, 1801] bf16 4.6 / 5.1, fp32 4.7 / 4.9, [1024, 1801] 6.5 / 5.4 and 6.6 / 5.7,
+// [16, 50257] 4.4 / 5.2 and 4.5 / 4.5, [128, 20001] 7.4 / 5.7 and 7.5 / 6.4.
+inline bool bwd_ragged_packs(int64_t rows, int64_t cols, int elem) {
+  if (cols * elem < 16) return false;
+  if (cols < kFlatPer) return rows > 6000;
+  return rows * cols >= (int64_t)3 << 19;
 }
 
 int check_xent(const char* what, int64_t rows, int64_t cols) {
@@ -320,7 +389,7 @@ extern "C" int eg_cross_entropy_fwd(const void* logits, const int64_t* target, v
       if (cols % V == 0 && aligned16(logits)) {
         pick_row_block(cols / V, LseLaunch<T, V>{xp, target, lse, rowloss, rows, (int)cols,
                                                  ignore_index, st});
-      } else if (cols >= V) {
+      } else if (fwd_ragged_packs(cols)) {
         pick_row_block((cols + V - 1) / V, LseLaunch<T, V, true>{xp, target, lse, rowloss, rows,
                                                                  (int)cols, ignore_index, st});
       } else {
@@ -363,7 +432,7 @@ extern "C" int eg_cross_entropy_bwd(const void* dloss, const void* logits,
     if (cols % V == 0 && aligned16(logits) && aligned16(dlogits))
       launch_bwd<T, T, T, V>(gp, xp, target, lse, n_valid, dp, rows, (int)cols, ignore_index,
                              st);
-    else if (cols >= V)
+    else if (bwd_ragged_packs(rows, cols, sizeof(T)))
       launch_bwd<T, T, T, V, true>(gp, xp, target, lse, n_valid, dp, rows, (int)cols,
                                    ignore_index, st);
     else
@@ -384,7 +453,7 @@ extern "C" int eg_cross_entropy_bwd(const void* dloss, const void* logits,
 //   losses and unit dlogits = softmax - onehot in place (one chunk of all rows by
 //   default: no fp32 logits are held);
 //   fp32 inputs: logits = x_c W^T (fp32) -> lse and row losses (xent_lse_kernel)
-//   -> unit dlogits (xent_bwd_flat_kernel), chunks of at most 2^29 logits;
+//   -> unit dlogits (launch_bwd), chunks of at most 2^29 logits;
 // then dx_c = dl_c W and dW (+)= dl_c^T x_c (MFMA; with more than one chunk the
 // products accumulate in an fp32 [vocab, hidden] buffer, added in each product's
 // epilogue, and the last chunk's product rounds the sum once into dW; fp32 inputs
@@ -771,24 +840,26 @@ extern "C" int eg_flce_fwd(const void* x, const void* weight, const int64_t* tar
                                  nullptr, 0, 0, rows))
           return rc;
         const float* none = nullptr;
-        if (vocab % 4 == 0) {
+        if (vocab % 4 == 0)
           pick_row_block(vocab / 4, LseLaunch<float, 4>{logits, target + r0, lse + r0,
                                                         rowloss + r0, n, (int)vocab,
                                                         ignore_index, st});
-          launch_bwd<float, T, float, 4>(none, logits, target + r0, lse + r0, nullptr, dlp, n,
-                                         (int)vocab, ignore_index, st, L.vp);
-        } else if (vocab >= 4) {
+        else if (fwd_ragged_packs(vocab))
           pick_row_block((vocab + 3) / 4, LseLaunch<float, 4, true>{logits, target + r0, lse + r0,
                                                                     rowloss + r0, n, (int)vocab,
                                                                     ignore_index, st});
-          launch_bwd<float, T, float, 4, true>(none, logits, target + r0, lse + r0, nullptr, dlp,
-                                               n, (int)vocab, ignore_index, st, L.vp);
-        } else {
+        else
           pick_row_block(vocab, LseLaunch<float, 1>{logits, target + r0, lse + r0, rowloss + r0,
                                                     n, (int)vocab, ignore_index, st});
+        if (vocab % 4 == 0)
+          launch_bwd<float, T, float, 4>(none, logits, target + r0, lse + r0, nullptr, dlp, n,
+                                         (int)vocab, ignore_index, st, L.vp);
+        else if (bwd_ragged_packs(n, vocab, 4))
+          launch_bwd<float, T, float, 4, true>(none, logits, target + r0, lse + r0, nullptr, dlp,
+                                               n, (int)vocab, ignore_index, st, L.vp);
+        else
           launch_bwd<float, T, float, 1>(none, logits, target + r0, lse + r0, nullptr, dlp, n,
                                          (int)vocab, ignore_index, st, L.vp);
-        }
         if (int rc = check_launch(name)) return rc;
       }
       // The partials of a split dx product go to memory that is free at this point: dW,

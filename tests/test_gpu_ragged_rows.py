@@ -106,3 +106,36 @@ def test_softmax_ragged_rows_in_place(rows, cols, dtype):
     _lib.call("eg_softmax_bwd", y.data_ptr(), over_dy.data_ptr(), over_dy.data_ptr(), *tail)
     _lib.call("eg_softmax_bwd", over_y.data_ptr(), dy.data_ptr(), over_y.data_ptr(), *tail)
     assert torch.equal(dx, over_dy) and torch.equal(dx, over_y)
+
+
+# Both sides of the lines between the backward's kernels (rows, flat with many rows or two per
+# workgroup; packs or single elements) and of the forward's: whole packs, then ragged.
+XENT_LINES = [(4095, 64, 0), (4096, 64, 0), (4096, 1280, 0), (4096, 1288, 0), (4097, 2048, 0),
+              (300, 4088, 0), (300, 8184, 0), (200, 8192, 0),
+              (6000, 9, 0), (6001, 9, 0), (6001, 255, 1), (6001, 897, 0), (6100, 1023, 3),
+              (1100, 1025, 0), (1534, 1025, 0), (1535, 1025, 0), (193, 8193, 0), (33, 50257, 0),
+              (70000, 5, 0)]
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("rows,cols,offset", XENT_LINES)
+def test_cross_entropy_rows_many(rows, cols, offset, dtype):
+    test_cross_entropy_ragged_rows(rows, cols, offset, dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+@pytest.mark.parametrize("rows,cols", [(6001, 33), (2000, 1277), (193, 8193), (5, 70), (4096, 64)])
+def test_cross_entropy_backward_in_place(rows, cols, dtype):
+    """dlogits over the logits gives the bits of separate buffers."""
+    print(f"\n[gpu-ragged] cross_entropy in place {rows}x{cols} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(rows, cols, device="cuda", generator=g).to(dtype)
+    t = torch.randint(0, cols, (rows,), device="cuda", generator=g)
+    lse = torch.logsumexp(x.float(), -1)
+    up, n = torch.ones((), device="cuda", dtype=dtype), torch.full((1,), float(rows), device="cuda")
+    dx, z = torch.empty_like(x), x.clone()
+    for a, b in ((x, dx), (z, z)):
+        _lib.call("eg_cross_entropy_bwd", up.data_ptr(), a.data_ptr(), t.data_ptr(),
+                  lse.data_ptr(), n.data_ptr(), b.data_ptr(), rows, cols, -100,
+                  _lib.dtype_tag(dtype), _lib.stream_of(x))
+    assert torch.equal(dx, z)
