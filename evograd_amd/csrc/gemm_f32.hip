@@ -11,7 +11,10 @@
 //   k-contiguous operand: row l%16 of each 16-row block, k = 4g .. +3 as one 16-byte load;
 //   k-major operand: rows k = 4g + e, TW columns TW (l%16) .. as one load, column
 //     TW (l%16) + j being row l%16 of block j.
-// Both put k = 4g + e in MFMA step e.
+// Both put k = 4g + e in MFMA step e. Operands whose rows or sizes are not whole aligned
+// 16-byte pieces take the same loads unaligned, and single elements in the last block of k
+// only (Run): element by element throughout, such products ran slower than one fed from LDS
+// (1435 x 1571 x 1933 644 us, now 178; 1577 x 4454 x 79 59, now 27).
 //
 // What bounds it: the MFMA rate where the output fills the chip, else the length of one
 // wave's k chain. Three tilings of a 256-thread workgroup, by the output's size alone:
@@ -38,13 +41,27 @@ struct F32Op {
   int64_t ld, rows;  // rows at or past `rows` read as zero
 };
 
+// How a run of an operand's elements is read: as one aligned load, as one load of any
+// alignment that may run up to three elements past a row's columns (into the rest of the
+// operand, so not in its last row: f32_whole), or element by element.
+enum class Run { kAligned, kAny, kElements };
+template <int W>
+using F32Run = float __attribute__((ext_vector_type(W)));
+template <int W, Run RUN>
+__device__ __forceinline__ F32Run<W> f32_run(const float* p) {
+  typedef F32Run<W> __attribute__((aligned(4))) any;
+  if constexpr (RUN == Run::kAligned) return *reinterpret_cast<const F32Run<W>*>(p);
+  else return *reinterpret_cast<const any*>(p);
+}
+
 // The 16 TW rows (or columns) of an operand from r0, k block k0 .. k0 + 15, as MFMA
-// operand values: f[j][e] for block j, step e. `ext` is M or N. VEC: 16-byte aligned rows,
+// operand values: f[j][e] for block j, step e. `ext` is M or N. kAligned: 16-byte aligned rows,
 // with K (k-contiguous) or ext (k-major) a multiple of 4, so every load lies inside or
-// outside the operand as a whole.
-template <bool KC, int TW, bool VEC>
+// outside the operand as a whole. What is read past ext is no output's operand.
+template <bool KC, int TW, Run RUN>
 __device__ __forceinline__ void f32_block(const F32Op& o, int r0, int k0, int ext, int K, int m16,
                                           int g, float (&f)[TW][4]) {
+  constexpr bool AL = RUN == Run::kAligned;
   if constexpr (KC) {
     const int k = k0 + 4 * g;
 #pragma unroll
@@ -52,9 +69,9 @@ __device__ __forceinline__ void f32_block(const F32Op& o, int r0, int k0, int ex
       const int64_t r = r0 + 16 * j + m16;
       const bool in = r < o.rows;
       const float* row = o.p + (in ? r : 0) * o.ld;
-      if constexpr (VEC) {
-        const bool ok = in && k < K;
-        const f32x4 x = *reinterpret_cast<const f32x4*>(row + (k < K ? k : 0));
+      if constexpr (RUN != Run::kElements) {
+        const bool ok = in && (!AL || k < K);
+        const f32x4 x = f32_run<4, RUN>(row + (!AL || k < K ? k : 0));
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[j][e] = ok ? x[e] : 0.f;
       } else {
@@ -73,12 +90,10 @@ __device__ __forceinline__ void f32_block(const F32Op& o, int r0, int k0, int ex
       const int64_t k = k0 + 4 * g + e;
       const bool in = k < o.rows;
       const float* row = o.p + (in ? k : 0) * o.ld;
-      if constexpr (VEC) {
-        typedef float fv __attribute__((ext_vector_type(TW)));
-        const bool ok = in && c < ext;
-        const fv x = *reinterpret_cast<const fv*>(row + (c < ext ? c : 0));
+      if constexpr (RUN != Run::kElements) {
+        const F32Run<TW> x = f32_run<TW, RUN>(row + (c < ext ? c : 0));
 #pragma unroll
-        for (int j = 0; j < TW; ++j) f[j][e] = ok ? x[j] : 0.f;
+        for (int j = 0; j < TW; ++j) f[j][e] = in ? x[j] : 0.f;
       } else {
 #pragma unroll
         for (int j = 0; j < TW; ++j) {
@@ -91,16 +106,24 @@ __device__ __forceinline__ void f32_block(const F32Op& o, int r0, int k0, int ex
   }
 }
 
+// Depth up to which an operand can be read as Run::kAny: a k-contiguous one to its last whole
+// run, a k-major one up to its last row, whose columns end the operand.
+template <bool KC>
+__device__ __forceinline__ int64_t f32_whole(const F32Op& o, int ext, int K) {
+  if (KC) return K;
+  return o.ld >= 4 && ext >= 4 ? (o.rows < K ? o.rows : (int64_t)K) - 1 : 0;
+}
+
 // Four columns of row `row` from `col`, plus the residual's.
 __device__ __forceinline__ void f32_store(float* C, int64_t ldc, const float* R,
-                                          int64_t ldr, int M, int N, int row, int col, bool vec,
-                                          f32x4 v) {
+                                          int64_t ldr, int M, int N, int row, int col, f32x4 v) {
+  typedef f32x4 __attribute__((aligned(4))) any4;
   if (row >= M) return;
   float* c = C + (int64_t)row * ldc + col;
   const float* r = R ? R + (int64_t)row * ldr + col : nullptr;
-  if (vec && col + 3 < N) {
-    if (r) v += *reinterpret_cast<const f32x4*>(r);
-    *reinterpret_cast<f32x4*>(c) = v;
+  if (col + 3 < N) {
+    if (r) v += *reinterpret_cast<const any4*>(r);
+    *reinterpret_cast<any4*>(c) = v;
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -115,7 +138,7 @@ template <bool AKC, bool BKC, int TW, bool CUT, bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, float* C, int M, int N,
                                                           int K, int64_t ldc, const float* R,
                                                           int64_t ldr, int tiles_n, int per,
-                                                          bool vec_c, float* part) {
+                                                          float* part) {
   constexpr int KU = TW == 2 ? 2 : 1;  // 16-deep k blocks per step
   constexpr int BT = CUT ? 16 * TW : 32 * TW;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -132,12 +155,21 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, floa
 #pragma unroll
     for (int j = 0; j < TW; ++j) acc[i][j] = f32x4{};
   float fa[2][KU][TW][4], fb[2][KU][TW][4];
-  auto load = [&](int set, int kb) {
+  auto load_as = [&](auto run, int set, int kb) {
+    constexpr Run R = decltype(run)::value;
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
-      f32_block<AKC, TW, VEC>(a, wm, 16 * (KU * kb + u), M, K, m16, g, fa[set][u]);
-      f32_block<BKC, TW, VEC>(b, wn, 16 * (KU * kb + u), N, K, m16, g, fb[set][u]);
+      f32_block<AKC, TW, R>(a, wm, 16 * (KU * kb + u), M, K, m16, g, fa[set][u]);
+      f32_block<BKC, TW, R>(b, wn, 16 * (KU * kb + u), N, K, m16, g, fb[set][u]);
     }
+  };
+  // without VEC: the k blocks before `whole` in unaligned loads, the last ones by elements
+  const int64_t depth = VEC ? 0 : min(f32_whole<AKC>(a, M, K), f32_whole<BKC>(b, N, K));
+  const int whole = (int)(depth / (16 * KU));
+  auto load = [&](int set, int kb) {
+    if constexpr (VEC) load_as(std::integral_constant<Run, Run::kAligned>{}, set, kb);
+    else if (kb < whole) load_as(std::integral_constant<Run, Run::kAny>{}, set, kb);
+    else load_as(std::integral_constant<Run, Run::kElements>{}, set, kb);
   };
   auto mul = [&](int set) {
 #pragma unroll
@@ -180,7 +212,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, floa
       f32x4 s = *reinterpret_cast<const f32x4*>(&buf[0][r][d]);
 #pragma unroll
       for (int k = 1; k < 4; ++k) s += *reinterpret_cast<const f32x4*>(&buf[k][r][d]);
-      f32_store(out, ldo, res, ldr, M, N, m0 + r, n0 + d, vec_c, s);
+      f32_store(out, ldo, res, ldr, M, N, m0 + r, n0 + d, s);
     }
   } else {
 #pragma unroll
@@ -189,7 +221,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, floa
       if constexpr (BKC) {
 #pragma unroll
         for (int j = 0; j < TW; ++j)
-          f32_store(out, ldo, res, ldr, M, N, row, wn + 16 * j + 4 * g, vec_c, acc[i][j]);
+          f32_store(out, ldo, res, ldr, M, N, row, wn + 16 * j + 4 * g, acc[i][j]);
       } else {
         // columns TW (4g + r) + j: 4 TW consecutive ones from 4 TW g
 #pragma unroll
@@ -197,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(F32Op a, F32Op b, floa
           f32x4 v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = acc[i][(4 * c + e) % TW][(4 * c + e) / TW];
-          f32_store(out, ldo, res, ldr, M, N, row, wn + 4 * TW * g + 4 * c, vec_c, v);
+          f32_store(out, ldo, res, ldr, M, N, row, wn + 4 * TW * g + 4 * c, v);
         }
       }
     }
@@ -266,13 +298,12 @@ int gemm_f32_launch(const float* A, const float* B, float* C, int64_t M, int64_t
   const bool vb = aligned16(B) && ldb % 4 == 0 && (b_kc ? K : N) % 4 == 0;
   float* part = p.splits > 1 ? (float*)ws : nullptr;
   const bool vr = !R || (aligned16(R) && ldr % 4 == 0);
-  const bool vec_c = part ? N % 4 == 0 : aligned16(C) && ldc % 4 == 0 && vr;
   auto go = [&](auto akc, auto bkc, auto tw, auto cut, auto vec) {
     EG_LAUNCH((gemm_f32_kernel<decltype(akc)::value, decltype(bkc)::value, decltype(tw)::value,
                                decltype(cut)::value, decltype(vec)::value>),
               dim3((unsigned)p.tiles, (unsigned)p.splits), dim3(256), 0, st,
               F32Op{A, lda, a_rows}, F32Op{B, ldb, b_rows}, C, (int)M, (int)N, (int)K, ldc, R, ldr,
-              tiles_n, (int)per, vec_c, part);
+              tiles_n, (int)per, part);
   };
   using TT = std::true_type;
   using FF = std::false_type;

@@ -51,3 +51,14 @@ def test_gemm_f32_splits_small_outputs_only():
     assert q(64, 40, 1001) == 4 * 64 * 40 * 4      # 4 tiles, 32 k steps: 4 splits
     assert q(33, 70, 100) == 0                     # 4 k steps
     assert q(512, 512, 4096) == 0                  # 256 tiles of 32
+
+
+# Each tiling where neither operand comes in whole aligned pieces: the last block of k alone,
+# after others, one element past them; outputs narrower than a load.
+@pytest.mark.parametrize("pad", (0, 1))
+@pytest.mark.parametrize("akc,bkc", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M,N,K", [(70, 35, 31), (70, 35, 65), (3, 2, 1025), (2, 3000, 50),
+                                   (1001, 1026, 31), (1001, 1026, 97), (2050, 2003, 15),
+                                   (2050, 2003, 49), (9000, 511, 33)])
+def test_gemm_f32_ragged(M, N, K, akc, bkc, pad):
+    test_gemm_f32(M, N, K, akc, bkc, pad)
