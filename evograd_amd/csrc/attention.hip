@@ -1154,21 +1154,26 @@ inline unsigned grid_for(int64_t BH, int nblocks) {
 // Two key groups per workgroup (KG = 2) in the forward and dQ: for grids of at most 512
 // 128-row workgroups, where the chain of key tiles of the last rows sets the time, from
 // 768 positions (12 tiles) on. bf16 forward / backward, one group against two: [1, 16 / 4,
-// 2000, 128] 38.2 / 116.9 -> 31.8 / 108.1 us, [1, 4 / 2, 4096, 128] 69.7 / 167.4 -> 54.9 /
-// 145.1, [1, 4, 8192, 64] 107.3 / 225.8 -> 89.0 / 207.2; shorter rows only pay for the
-// exchange ([1, 2 / 1, 200, 128] 8.2 -> 9.0 us, [4, 8, 512, 128] 12.8 -> 13.3).
+// 2000, 128] 38.0 / 114.4 -> 30.7 / 108.5 us, [1, 4, 900, 128] 19.7 / 51.3 -> 17.7 / 50.7, [1, 8,
+// 768, 64] 13.0 / 33.9 -> 12.0 / 34.0; shorter rows only pay for the exchange ([1, 2 / 1, 200,
+// 128] 8.2 -> 9.0 us, [4, 8, 512, 128] 12.8 -> 13.3).
 // A CU holds one workgroup of two groups or two of one, so past 256 workgroups the second
-// round has to be won back by longer rows: forward at D = 128 [1, 64 / 8, 1000] 28.0 -> 30.1
-// us but [1, 32 / 8, 2048] 46.7 -> 43.9, at 64 always ahead ([1, 40 / 8, 1000] 16.9 -> 15.5);
-// backward at 128 [1, 48 / 12, 903] 90.5 -> 97.0, [1, 32 / 8, 2048] 178.1 -> 180.9, but
-// [1, 24 / 8, 2048] 154.6 -> 151.3 and [1, 16 / 4, 4096] 290.4 -> 281.7, at 64 [1, 32 / 8,
-// 1800] (480 workgroups) 84.5 -> 85.2 but [2, 24 / 8, 1024] (384) 61.1 -> 59.5.
+// round has to be won back by longer rows. Forward: at D = 128 from 2048 positions ([1, 64 / 8,
+// 1000] 28.0 -> 30.1, [1, 32 / 8, 2048] 47.8 -> 44.5), at 64 always ([1, 64 / 8, 800] 16.2 -> 15.8,
+// [1, 40 / 8, 1152] 19.5 -> 17.9). dQ, backward: up to 384 workgroups at 128 from 2048 ([1, 24 /
+// 8, 2048] 150.4 -> 144.4, [1, 16 / 4, 2500] 146.3 -> 135.5, [1, 48 / 12, 903] 90.5 -> 97.0), at 64
+// from 1152 ([3, 16, 900] 50.4 -> 53.8, [2, 24, 780] 44.3 -> 47.3, [1, 40 / 8, 1152] 60.7 -> 60.6,
+// [1, 24 / 8, 2048] 86.0 -> 81.8); up to 512 from 4096 ([1, 32 / 8, 2048, 128] 173.4 -> 171.7 but
+// 178.1 -> 180.9 on another card, [1, 16 / 4, 4096, 128] 287.6 -> 273.5).
+// A head's result is a sum in the order its grid takes, so it may differ in its last bits
+// between calls with few and with many heads.
 constexpr int64_t kSplitKeysGrid = 512, kSplitKeysSeq = 768;
 inline bool split_keys(int64_t BH, int64_t S, int64_t D, bool dq) {
   const int64_t grid = grid_for(BH, (int)((S + 127) / 128));
   if (S < kSplitKeysSeq || grid > kSplitKeysGrid) return false;
-  const bool longer = D == 64 || S >= 2048;
-  return grid <= 256 || (dq ? S >= 4096 || (grid <= 384 && longer) : longer);
+  if (grid <= 256) return true;
+  if (!dq) return D == 64 || S >= 2048;
+  return S >= 4096 || (grid <= 384 && S >= (D == 64 ? 1152 : 2048));
 }
 
 // With ROPE, q is rotated in registers by the fp32 tables rc/rs [S, D] as it is

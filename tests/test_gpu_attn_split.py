@@ -71,3 +71,12 @@ def test_attention_split_is_bitwise_repeatable():
         o, saved = mod.causal_attention_gqa_forward_with_saved(q, k, v)
         runs.append((o, *mod.causal_attention_gqa_backward_from_saved(do, saved)))
     assert all(torch.equal(a, b) for a, b in zip(*runs))
+
+
+# On both sides of the lines for grids past 256 workgroups: dQ at 1152 positions (head size
+# 64) and 2048 (128), the forward at 2048 (128).
+@pytest.mark.parametrize("B,H,KVH,S,D", [(1, 40, 8, 1151, 64), (1, 40, 8, 1152, 64),
+                                         (3, 16, 16, 900, 64), (1, 24, 8, 2047, 128),
+                                         (1, 24, 8, 2048, 128)])
+def test_attention_split_keys_lines(B, H, KVH, S, D):
+    test_attention_split(B, H, KVH, S, D, "bfloat16")
