@@ -177,6 +177,8 @@ def layer_flops(d: dict) -> dict:
     return {"fwd": 2.0 * M * P + dense, "bwd": 4.0 * M * P + 5 * dense / 2}
 
 
+PRODUCTS = ("gemm_kernel", "gemm_mid_kernel", "gemm_f32_kernel")
+
 # The kernel whose roofline each op reports: (phase, kernel name, occurrence of that
 # name among the phase's launches), with its algorithmic work per launch from
 # dominant_work. Launch sequences are discovered by the timing hook (every launch
@@ -263,8 +265,10 @@ def kernel_times(name: str, fwd, bwd_call, setup_bwd, state, flush, steps: int) 
 
 
 def find_kernel(kt: dict, phase: str, kname: str, occurrence: int) -> str:
-    """Key of the occurrence-th launch of kernel kname in a phase."""
-    hits = [k for k in kt if k.split(":")[0] == phase and k.split(":")[2] == kname]
+    """Key of the occurrence-th launch of kernel kname in a phase. A product counts
+    whichever kernel its size gave it to."""
+    names = PRODUCTS if kname in PRODUCTS else (kname,)
+    hits = [k for k in kt if k.split(":")[0] == phase and k.split(":")[2] in names]
     if len(hits) <= occurrence:
         raise KeyError(f"{phase} has {len(hits)} launches of {kname}, not {occurrence + 1}")
     return hits[occurrence]

@@ -47,3 +47,17 @@ def test_traffic_calibrates_on_the_copy_grid_not_the_largest_reading(tmp_path):
     assert e["fetch_bytes_per_launch"] == round(1001.0 * 1024 * 2)
     assert e["write_bytes_per_launch"] == 500 * 1024
     assert e["hbm_bytes_per_launch"] == e["fetch_bytes_per_launch"] + e["write_bytes_per_launch"]
+
+
+def test_bench_finds_a_layers_products_on_either_kernel():
+    """The decoder layer reports its gate and up projections, the third product, whichever
+    kernels the products before it run on."""
+    import bench
+
+    kt = {k: 1.0 for k in ("fwd:0:rmsnorm_fwd_row", "fwd:1:gemm_kernel",
+                           "fwd:2:splitk_reduce_kernel", "fwd:3:attn_fwd_kernel",
+                           "fwd:4:gemm_mid_kernel", "fwd:5:gemm_kernel", "fwd:6:silu_mul_kernel",
+                           "fwd:7:gemm_kernel", "bwd:0:gemm_kernel")}
+    phase, name, occurrence = bench.DOMINANT["llama3_decoder_layer@llama3_8b_T1024"]
+    assert bench.find_kernel(kt, phase, name, occurrence) == "fwd:5:gemm_kernel"
+    assert bench.find_kernel(kt, "fwd", "silu_mul_kernel", 0) == "fwd:6:silu_mul_kernel"
