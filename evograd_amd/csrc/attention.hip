@@ -1092,9 +1092,9 @@ int dkdv_parts(int64_t BHkv, int64_t S, int64_t D) {
 // walk until the chip is full (two workgroups per CU) and costs its slabs' write and read.
 // In us, 1.1 (D = 128) or 0.9 (64) per 32-row step, 1.6 per million elements of dK and
 // part, and 5 for the reduction: fitted over 48 shapes timed at every number of parts; the
-// backward at the choice against at the bound: bf16 [2, 12, 1000, 64] 52.4 -> 44.6 us in 3
-// parts, [4, 8, 512, 128] 72.9 -> 45.8 in 1, [1, 8, 2048, 128] 106.6 -> 91.2 in 3 (88.0 in 4),
-// [1, 32 / 8, 512, 128] 46.8 in 8 (49.2 in 6), [1, 4, 8192, 64] 207.6 in 4 (241.9 in 2).
+// backward at the bound against at the choice: bf16 [2, 12, 1000, 64] 54.7 -> 46.4 us (6 parts,
+// 3), [4, 8, 512, 128] 72.1 -> 44.4 (8, 1), [1, 8, 2048, 128] 107.7 -> 92.2 (8, 5), [8, 16, 256, 64]
+// 40.9 -> 22.0 (4, 1); [1, 32 / 8, 512, 128] stays at 8 parts, [1, 4, 8192, 64] at 4.
 int dkdv_split(int64_t BHkv, int64_t group, int64_t S, int64_t D) {
   const int most = dkdv_parts(BHkv, S, D);
   const double step = D == 128 ? 1.1 : 0.9;

@@ -27,8 +27,9 @@
 // over the other side is cut over the kGenWaves waves of a workgroup (tile t to wave
 // t % kGenWaves), which add their parts through LDS in wave order; the dK/dV walk is
 // also cut over `parts` workgroups whose fp32 slabs attn_gen_reduce_kernel adds in
-// order. At fp32 [1, 8 / 2 kv, 1024, 64] the kernels take 22 us (forward), 33 us (dQ)
-// and 43 + 5 us (dK/dV and its reduction), against 6031, 6316 and 30931 us for one wave per
+// order. At fp32 [1, 8 / 2 kv, 1024, 64] a kernel trace has 21.5 us (forward), 32.6 (dQ) and
+// 42.6 + 4.7 (dK/dV and its reduction), with the matrix cores busy for 38% of the cycles of
+// each, against 6031, 6316 and 30931 us for one wave per
 // 64 rows on VALU FMAs (128 waves on the chip's 1024 SIMDs, about 6 us per key of the
 // longest row: one dependent chain with its operands broadcast from LDS).
 // No atomics: every sum has a fixed order.
@@ -190,9 +191,9 @@ inline dim3 gen_grid(int64_t x, int64_t blocks) {
 // so that what a CU takes last is short. PAIR, for kernels with two workgroups on a CU:
 // where the whole grid is resident at once (kGenTarget), nothing is taken last and the
 // second workgroup of each CU comes shortest first, so that every CU holds a long and a
-// short walk. fp32, longest first against paired: [1, 8 / 2 kv, 1024, 64] forward 23.6 ->
-// 19.7 us, backward 87.4 -> 73.0 (the longest CU had 1.5 times the mean work), [1, 8 / 2,
-// 1000, 128] forward 44.8 -> 37.2; the backward there has registers for one workgroup on
+// short walk. fp32 calls, longest first against paired: [1, 8 / 2 kv, 1024, 64] forward 26.2 ->
+// 22.1 us, backward 91.5 -> 77.0 (the longest CU had 1.5 times the mean work), [1, 8 / 2,
+// 1000, 128] forward 45.9 -> 36.9; the backward there has registers for one workgroup on
 // a CU and would go 176.6 -> 189.9.
 template <bool PAIR>
 __device__ __forceinline__ int walk_order(int blk, int n) {

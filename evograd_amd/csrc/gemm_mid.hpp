@@ -1,5 +1,5 @@
 // The 16-bit product of gemm_kernel.hpp on 128 x 128 x 64 tiles, for outputs that are too
-// small to occupy the chip in 256 x 256 tiles (the choice: gemm.hip, use_mid).
+// small to occupy the chip in 256 x 256 tiles (the choice: gemm.hip, gemm_plan).
 //
 // Same operands, layouts, segments, bounds and k order as gemm_kernel: fp32 accumulation on
 // v_mfma_f32_32x32x16 over 64-deep slices in increasing k, so a product's bits depend on

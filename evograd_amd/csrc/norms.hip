@@ -73,10 +73,14 @@ inline int64_t ring_blocks(int64_t rows, int64_t per512, int block) {
 // it read). Backward call, bf16, before and after: RMSNorm [4000, 512] 17.7 -> 10.5 us,
 // [8000, 1024] 21.2 -> 16.4, [16000, 512] 25.0 -> 17.7, [16000, 2048] 41.7 -> 38.0;
 // LayerNorm [4000, 1024] 21.3 -> 13.8, [65536, 512] 52.1 -> 44.0; 256 workgroups, or 4096
-// at 64 threads, are slower at each of these. fp32 rings of 256 threads keep the larger
-// count below 2048 rows ([1500, 1000]: 12.6 us against 10.6): the declared fp32 gate, 1e-5
-// against an fp32 oracle that is itself up to 1.2 times that off 64 bits at such sizes,
-// has no room there for another order of the same sums.
+// at 64 threads, are slower at each of these. Fewer workgroups add more rows each, at no cost
+// in precision: fp32 dweight against 64 bits over 13 widths up to 1024 and 12 row counts from
+// 257 to 16384, relative error 1.14e-7 on average and 1.59e-7 at most, 1.20e-7 and 1.63e-7 with
+// the larger counts. fp32 rings of 256 threads keep the larger count below 2048 rows
+// all the same, and give up 10-25% there ([1500, 1000] 15.0 us against 13.2): the declared fp32
+// gate compares with an fp32 oracle that is itself over the gate off 64 bits in some columns
+// at such sizes, so every order of these sums fails it somewhere, this one at no tested size.
+// Compensated sums (1.10e-7, 1.36e-7) pass it too but cost the larger calls 1-6%.
 inline int64_t bwd_ring_blocks(int64_t rows, int64_t per512, int block, int elem) {
   if (block >= 512 || (block == 256 && elem == 4 && rows < 2048))
     return ring_blocks(rows, per512, block);
@@ -844,7 +848,7 @@ __global__ __launch_bounds__(1024) void colsum_wide_kernel(const float* __restri
 }
 
 // 32 columns per workgroup (measured at 512 x 4096 partial rows: 7.9 us cold for
-// one parameter, 10.3 us for two, against 8.8 and 14.0 us for colsum_kernel).
+// one parameter, 10.3 us for two).
 constexpr int kColsumQuads = 8;
 
 template <typename T>
