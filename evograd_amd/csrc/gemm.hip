@@ -34,12 +34,19 @@ int gemm_splits(int64_t M, int64_t N, int64_t K) {
 // Which kernel a product of at most kSplitTarget / 2 tiles of 256 x 256 runs on, and its
 // split of k: the cheaper of the two by a cost in us fitted to both kernels over outputs
 // of 77-2048 x 256-28672 at depths 77-28672 (bf16, three layouts; within 15% of most).
-// A 256 x 256 workgroup costs 10 + 1.63 per 64-deep slice, a 128 x 128 one 5 + 0.62; 256
-// run at a time; a split adds its reduction, 8 + the partials at 5 TB/s. So the 128 x 128
-// kernel takes small outputs and short depths (77 x 256 x 256: 13.6 -> 6.8 us, 600 x 3584 x
-// 1024: 28.9 -> 15.2, 2048 x 2048 x 1024: 37.0 -> 16.1, 1024 x 4096 x 4096: 54.6 -> 42.9) and
-// the 256 x 256 one long depths (1024 x 4096 x 14336: 123 against 166) and every larger
-// output (2048 x 7168 x 1024, 224 tiles: 36 against 54).
+// A 256 x 256 workgroup costs 10 + 1.63 per 64-deep slice, a 128 x 128 one 5 + 0.62 with its
+// operands in cache; 32 run at a time on each of the eight XCDs, which take the tiles in turn
+// (50 tiles in 5 ranges are 35 workgroups on the first: a second round); a split adds its
+// reduction, 8 + the partials at 5 TB/s. Against the large tiles a slice of the 128 x 128
+// kernel counts 0.72: with operands in HBM, as a layer's weights are, its workgroups wait for
+// more of them, all at the same depth when k is not split. us, large tiles against 128 x 128,
+// operands in HBM and in cache: 1024 x 4096 x 6144 76 / 85 and 68 / 65, 256 x 11328 x 5312 74 / 88
+// and 54 / 58, 1024 x 4096 x 4096 66 / 65 and 58 / 49, 2048 x 2048 x 4096 59 / 57 and 54 / 46.
+// So the 128 x 128 kernel takes small outputs and short depths (77 x 256 x 256: 13.6 -> 6.8 us,
+// 600 x 3584 x 1024: 30.6 -> 17.2 in cache, 20.2 from HBM, 2048 x 2048 x 1024: 38.5 -> 17.9 and
+// 21.5), or what the large tiles cannot split evenly over the XCDs (256 x 4288 x 8256, 17 tiles in 15
+// ranges: 83 -> 60), and the 256 x 256 one long depths (1280 x 640 x 22144: 75 against 122) and
+// every larger output (2048 x 7168 x 1024, 224 tiles: 36 against 54).
 // The 128 x 128 kernel never takes more parts than gemm_splits, whose partials the
 // caller's workspace is sized for.
 struct GemmPlan {
@@ -49,25 +56,27 @@ struct GemmPlan {
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int max_splits, int fixed_splits) {
   auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
   const int64_t nk = (K + kBK - 1) / kBK, big = tiles(kBM), small = tiles(kMT);
+  constexpr int64_t kXcds = 8, kXcdCus = kSplitTarget / kXcds;
+  auto on_xcd = [&](int64_t t, int64_t s) { return (t + kXcds - 1) / kXcds * s; };
   auto cost = [&](int64_t t, double fixed, double slice, int64_t s) {
-    const int64_t waves = (t * s + kSplitTarget - 1) / kSplitTarget;
+    const int64_t waves = (on_xcd(t, s) + kXcdCus - 1) / kXcdCus;
     const double run = (double)waves * (fixed + slice * (double)((nk + s - 1) / s));
     return s > 1 ? run + 8.0 + (double)s * (double)M * (double)N * 4e-6 / 5.0 : run;
   };
   const int sb = fixed_splits > 0 ? fixed_splits : std::min(max_splits, gemm_splits(M, N, K));
-  GemmPlan best{false, sb};
-  if (big > kSplitTarget / 2) return best;
-  double least = cost(big, 10.0, 1.63, sb);
-  for (int s = fixed_splits > 0 ? fixed_splits : 1; s <= sb; ++s) {
-    if (fixed_splits <= 0 && s > 1 && small * s > kSplitTarget) break;
+  const GemmPlan large{false, sb};
+  if (big > kSplitTarget / 2) return large;
+  GemmPlan best{true, fixed_splits > 0 ? fixed_splits : 1};
+  double least = cost(small, 5.0, 0.62, best.splits);
+  for (int s = 2; fixed_splits <= 0 && s <= sb && on_xcd(small, s) <= kXcdCus; ++s) {
     const double c = cost(small, 5.0, 0.62, s);
     if (c < least) {
       const int64_t per = (nk + s - 1) / s;
       least = c;
-      best = GemmPlan{true, fixed_splits > 0 ? s : (int)((nk + per - 1) / per)};
+      best.splits = (int)((nk + per - 1) / per);
     }
   }
-  return best;
+  return cost(small, 5.0, 0.72, best.splits) < cost(big, 10.0, 1.63, sb) ? best : large;
 }
 int gemm_plan_splits(int64_t M, int64_t N, int64_t K, int dtype) {
   return dtype == EG_F32 ? gemm_f32_splits(M, N, K) : gemm_plan(M, N, K, kMaxSplits, 0).splits;

@@ -304,7 +304,7 @@ LARGE = [
     # more than 128 tiles, unsplit, ragged in M, N and (k-major) K
     *((2900, 3000, 320, *lay) for lay in LAYOUTS), (2900, 3000, 100, False, False),
     # split k, ragged likewise
-    *((1000, 4000, 14336, *lay) for lay in LAYOUTS), (700, 3001, 9000, False, False),
+    *((1000, 4000, 14336, *lay) for lay in LAYOUTS), (900, 3001, 14300, False, False),
 ]
 
 

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from evograd_amd import _lib
+from evograd_amd.timing import KernelTimer
 
 pytestmark = pytest.mark.gpu
 ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
@@ -78,3 +79,25 @@ def test_gemm_mid_bits_equal_the_large_tiles(akc, bkc):
     _product(a, b, whole, None, M, N, K, akc, bkc, torch.bfloat16, 0)
     _product(few, b, part, None, m, N, K, akc, bkc, torch.bfloat16, 0)
     assert torch.equal(whole[:m], part)
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (1024, 4096, 4096, "gemm_mid_kernel"), (1024, 4096, 6144, "gemm_kernel"),
+    (1280, 640, 22144, "gemm_kernel"),      # 50 small tiles in 5 ranges: 35 on one XCD
+    (700, 3001, 9024, "gemm_mid_kernel"),   # 36 large tiles in 7 ranges: likewise
+    (640, 1152, 4096, "gemm_mid_kernel")])  # 45 small tiles, split
+def test_product_kernel_by_size(M, N, K, kernel):
+    """The lines of the choice between the two kernels, and its products against fp64."""
+    print(f"\n[gpu-gemm-mid] {M}x{N}x{K} on {kernel}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    b = torch.randn(N, K, device="cuda", generator=g).bfloat16()
+    c = torch.empty(M, N, device="cuda", dtype=torch.float32)
+    need = _lib.query("eg_gemm_workspace_bytes", M, N, K, _lib.EG_BF16)
+    timer = KernelTimer()
+    timer.arm(0)
+    _product(a, b, c, None, M, N, K, True, True, torch.bfloat16, need)
+    assert timer.label() == kernel
+    timer.close()
+    A, B = a.double(), b.double().t()
+    assert ((c.double() - A @ B).abs() <= (K + 20) * 2.0 ** -24 * (A.abs() @ B.abs())).all()
