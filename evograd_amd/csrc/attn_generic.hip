@@ -27,8 +27,8 @@
 // over the other side is cut over the kGenWaves waves of a workgroup (tile t to wave
 // t % kGenWaves), which add their parts through LDS in wave order; the dK/dV walk is
 // also cut over `parts` workgroups whose fp32 slabs attn_gen_reduce_kernel adds in
-// order. At fp32 [1, 8 / 2 kv, 1024, 64] a kernel trace has 21.5 us (forward), 32.6 (dQ) and
-// 42.6 + 4.7 (dK/dV and its reduction), with the matrix cores busy for 38% of the cycles of
+// order. At fp32 [1, 8 / 2 kv, 1024, 64] a kernel trace has 21.1 us (forward), 32.2 (dQ) and
+// 41.7 + 4.7 (dK/dV and its reduction), with the matrix cores busy for 38% of the cycles of
 // each, against 6031, 6316 and 30931 us for one wave per
 // 64 rows on VALU FMAs (128 waves on the chip's 1024 SIMDs, about 6 us per key of the
 // longest row: one dependent chain with its operands broadcast from LDS).
