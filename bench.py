@@ -29,6 +29,11 @@ T in {1024, 2048, 4096} at Llama-3-8B widths, with its MFMA fraction over the
 layer's model FLOPs. ``sweeps`` holds the memory-bound operators over the
 reference's token sweeps (src/evograd/opdecl/models.py:286, :293).
 
+stdout gets one JSON line: the headline and, for each operator, its latencies,
+roofline fractions, saved bytes, dominant kernel and speedups. What lies behind them
+(every kernel's time, every saved tensor, quantiles, bytes and FLOPs) goes to stderr
+first, one ``detail`` line per operator, so that the result line stays a few KB.
+
 Each operator with an eager spelling also reports ``gpu_eager_full_us``: the reference's
 eager forward (torch operators) plus torch autograd on the same GPU and inputs, and
 ``speedup_vs_gpu_eager``. ``sustained`` holds the device's sustained MFMA and copy rates
@@ -99,6 +104,36 @@ def bench_workload(op, label: str):
 
 def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def rounded(v, digits: int = 5):
+    """`v` with every float in it cut to `digits` significant digits."""
+    if isinstance(v, float):
+        return float(f"{v:.{digits}g}")
+    if isinstance(v, dict):
+        return {k: rounded(x, digits) for k, x in v.items()}
+    return v
+
+
+def op_summary(r: dict) -> dict:
+    """What the result line holds of one operator; the whole of `r` goes to stderr."""
+    if "error" in r:
+        return {"error": r["error"][:200]}
+    out = {k: r[k] for k in ("fwd_us", "bwd_us", "full_us", "hbm_frac_full", "mfma_frac_full",
+                             "mfma_frac_full_of_sustained", "speedup_vs_gpu_eager",
+                             "speedup_vs_cpu") if k in r}
+    out["saved_bytes"] = r["saved"]["logical_saved_bytes"]
+    dk = r.get("dominant_kernel")
+    if dk:
+        out["kernel"] = {k: dk[k] for k in ("name", "us", "frac") if k in dk}
+    return rounded(out)
+
+
+def sweep_summary(s: dict) -> dict:
+    """Latency in us and HBM fraction at each point of one operator's sweep."""
+    if "error" in s:
+        return {"error": str(s["error"])[:200]}
+    return {t: [v["full_us"], v["hbm_frac_full"]] for t, v in s.items()}
 
 
 # ------------------------------------------------------------ algorithmic work
@@ -980,9 +1015,13 @@ def main() -> int:
                          if HEADLINE in cpu and "value" in cpu[HEADLINE] else None),
         "cpu_model": cpu_model(),
         "sustained": sustained,
-        "ops": results,
-        "sweeps": sweeps,
+        "ops": {k: op_summary(r) for k, r in results.items()},
+        "sweeps": {k: sweep_summary(v) for k, v in sweeps.items()},
     }
+    for name, r in results.items():
+        log(f"detail {name}: " + json.dumps(r))
+    for name, r in sweeps.items():
+        log(f"detail sweep {name}: " + json.dumps(r))
     traffic = load_traffic("norm_bwd_ring")
     if traffic is not None:
         line["roofline"]["traffic"] = traffic.get("hbm_bytes_per_launch")

@@ -61,3 +61,28 @@ def test_bench_finds_a_layers_products_on_either_kernel():
     phase, name, occurrence = bench.DOMINANT["llama3_decoder_layer@llama3_8b_T1024"]
     assert bench.find_kernel(kt, phase, name, occurrence) == "fwd:5:gemm_kernel"
     assert bench.find_kernel(kt, "fwd", "silu_mul_kernel", 0) == "fwd:6:silu_mul_kernel"
+
+
+def test_bench_line_leaves_the_details_out():
+    """The result line's share of one operator is its figures, whatever the number of
+    kernels and saved tensors behind them, and an operator that failed keeps its error."""
+    import json
+
+    import bench
+
+    r = {"config": {"dims": {"T": 1024}, "dtype": "bfloat16"}, "fwd_us": 555.0900001,
+         "bwd_us": 1450.4, "full_us": 1947.8, "mfma_frac_full": 0.27951234,
+         "saved": {"logical_saved_bytes": 462053376, "ratio_to_memory_inputs": 1.5},
+         "saved_tensors": [{"kind": "tensor", "shape": [1024, 4096]}] * 40,
+         "kernels_us": {f"bwd:{i}:gemm_kernel": 200.123456789 for i in range(60)},
+         "dominant_kernel": {"name": "fwd:8:gemm_kernel", "phase": "fwd", "us": 209.891234,
+                             "flops": 1, "frac": 0.45534}}
+    out = bench.op_summary(r)
+    assert out == {"fwd_us": 555.09, "bwd_us": 1450.4, "full_us": 1947.8,
+                   "mfma_frac_full": 0.27951, "saved_bytes": 462053376,
+                   "kernel": {"name": "fwd:8:gemm_kernel", "us": 209.89, "frac": 0.45534}}
+    assert len(json.dumps(out)) < 400
+    assert bench.op_summary({"error": "RuntimeError: x"}) == {"error": "RuntimeError: x"}
+    sweep = {"256": {"full_us": 13.1, "hbm_frac_full": 0.1, "kernels_us": {"k": 4.0}}}
+    assert bench.sweep_summary(sweep) == {"256": [13.1, 0.1]}
+    assert bench.sweep_summary({"error": "e"}) == {"error": "e"}
