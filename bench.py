@@ -1,11 +1,10 @@
 #!/usr/bin/env python3
 """Benchmark of the autograd-pair hot path on one MI355X.
 
-Metric (BASELINE.json): fwd+bwd step latency (us) + % HBM/MFMA roofline per op;
+Metric: fwd+bwd step latency (us) + % HBM/MFMA roofline per op;
 saved bytes vs CPU. The headline ``value`` is the full-step (forward + backward)
-latency of RMSNorm bf16 x[16384, 4096], eps 1e-6; every other
-BASELINE configuration is measured the same way and reported under ``ops``, with the
-operators beyond BASELINE at their declared benchmark workloads. ``op@label``
+latency of RMSNorm bf16 x[16384, 4096], eps 1e-6; every other operator is measured the
+same way at its declared benchmark workload and reported under ``ops``. ``op@label``
 selects another labelled benchmark workload of an operator (``softmax@vocab``: bf16
 rows of the Llama-3 vocabulary, the reference's timed default width).
 
@@ -802,7 +801,7 @@ COPY_BYTES = 256 << 20
 
 def profile_run(name: str, steps: int) -> dict:
     """Workload for rocprofv3: ``steps`` x (cache flush, forward, backward) of one
-    operator at its BASELINE configuration, then ``steps`` plain copies of
+    operator at its benchmark workload, then ``steps`` plain copies of
     COPY_BYTES (a torch elementwise kernel reading and writing COPY_BYTES each),
     whose FETCH_SIZE/WRITE_SIZE readings calibrate the counters for the op's
     kernels."""
@@ -995,8 +994,7 @@ def main() -> int:
         "dtype": "bf16",
         "data": "synthetic",
         "config": {
-            "workload": f"rmsnorm fwd+bwd bf16 x[{dims['rows']},{dims['hidden']}] eps=1e-6 "
-                        "(BASELINE configs[1])",
+            "workload": f"rmsnorm fwd+bwd bf16 x[{dims['rows']},{dims['hidden']}] eps=1e-6",
             "rows": dims["rows"], "hidden": dims["hidden"],
             "parallelism": "single-gpu",
         },
